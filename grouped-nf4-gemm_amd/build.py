@@ -1,7 +1,7 @@
 """Build libgnf4_hip.so in-tree for gfx950 with hipcc.
 
 ``python build.py`` (or ``build()``) compiles the HIP sources in csrc/ (the
-grouped GEMM kernels and the routing kernels) into ``libgnf4_hip.so`` next to
+grouped GEMM kernels, its tile kernels and the routing kernels) into ``libgnf4_hip.so`` next to
 this file, and the measurement kernels bench.py times against
 (``csrc/gnf4_floor.hip``) into ``libgnf4_floor.so``. It always recompiles: the library must
 track its source, and the GPU box only ever loads the prebuilt file.
@@ -11,10 +11,12 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
-SRCS = [HERE / "csrc" / "gnf4_hip.hip", HERE / "csrc" / "gnf4_route.hip"]
+SRCS = [HERE / "csrc" / n for n in ("gnf4_hip.hip", "gnf4_tile.hip", "gnf4_route.hip")]
 OUT = HERE / "libgnf4_hip.so"
 FLOOR_SRCS = [HERE / "csrc" / "gnf4_floor.hip"]
 FLOOR_OUT = HERE / "libgnf4_floor.so"
@@ -23,7 +25,7 @@ ARCH = os.environ.get("GNF4_HIP_ARCH", "gfx950")
 # -packed-fp32-ops: keep the compiler from emitting v_pk_{add,mul,fma}_f32 for
 # ordinary float code (this build targets boxes where those forms are avoided).
 HIPCC_FLAGS = [
-    "-O3", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", f"--offload-arch={ARCH}",
+    "-O3", "-std=c++17", "-ffp-contract=off", "-fPIC", f"--offload-arch={ARCH}",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
@@ -36,10 +38,8 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found (set HIPCC)")
 
 
-def _compile(srcs, out: Path, verbose: bool) -> Path:
-    tmp = out.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-o", str(tmp), *(str(p) for p in srcs)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+def _hipcc(args, verbose: bool) -> None:
+    r = subprocess.run([hipcc(), *HIPCC_FLAGS, *args], capture_output=True, text=True)
     # hipcc's host pass does not know the packed-fp32 feature and says so.
     noise = "is not a recognized feature for this target"
     msgs = "\n".join(l for l in (r.stdout + r.stderr).splitlines() if noise not in l)
@@ -47,6 +47,17 @@ def _compile(srcs, out: Path, verbose: bool) -> Path:
         raise RuntimeError(f"hipcc failed ({r.returncode}):\n{msgs}")
     if verbose and msgs.strip():
         print(msgs)
+
+
+def _compile(srcs, out: Path, verbose: bool) -> Path:
+    """One object per source, compiled at the same time, linked into `out`."""
+    tmp = out.with_suffix(".so.tmp")
+    with tempfile.TemporaryDirectory() as d:
+        objs = [str(Path(d) / (p.stem + ".o")) for p in srcs]
+        with ThreadPoolExecutor(len(srcs)) as pool:
+            list(pool.map(lambda so: _hipcc(["-c", str(so[0]), "-o", so[1]], verbose),
+                          zip(srcs, objs)))
+        _hipcc(["-shared", "-o", str(tmp), *objs], verbose)
     os.replace(tmp, out)
     return out
 

@@ -54,355 +54,12 @@
 #include <mutex>
 #include <type_traits>
 
-#include "../../include/gnf4_hip.h"
+#include "gnf4_device.h"
+#include "gnf4_tile.h"
+
+using namespace gnf4;
 
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
-typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
-typedef __attribute__((ext_vector_type(2))) int v2i32_t;
-
-constexpr int kNF4 = GNF4_FMT_NF4;
-constexpr int kMX = GNF4_FMT_MXFP4;
-
-// NF4 codebook, reference kernel/nf4_grouped.py:53-70 (code 7 is exactly 0).
-__constant__ float c_nf4[16] = {
-    -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
-    -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
-    0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f,
-    0.33791524171829224f, 0.44070982933044434f, 0.5626170039176941f,
-    0.7229568362236023f, 1.0f,
-};
-
-// ---------------------------------------------------------------- decode --
-
-// The NF4 pair table: 256 bytes x 32 lane columns x float2 = 64 KiB. Entry
-// (byte, column) holds the fp32 pair (NF4[byte >> 4], NF4[byte & 15]) in the
-// column of lane % 32, so the lanes one LDS pass serves read distinct banks.
-// Declared first so it sits at LDS offset 0: one v_perm_b32 then forms the
-// full address byte << 8 | (lane % 32) * 8.
-constexpr int kPairEntries = 256 * 32;
-
-// Codebook entry `lane % 16` in one register per lane. Kernels load it before
-// any weight load: vector loads complete in order, so a codebook read issued
-// after the weights would hold the table build until every weight landed.
-__device__ __forceinline__ int nf4_lut_lane() {
-  return __float_as_int(c_nf4[threadIdx.x & 15]);
-}
-
-__device__ __forceinline__ void init_pair_table(float2* tab, int lut) {
-  // Thread t fills the columns of byte t % 256 (all 32 of them with 256
-  // threads, half of them with 512), rotating the column order by byte so one store instruction
-  // touches distinct banks. Entries come from the codebook register of lanes
-  // 0..15 through ds_bpermute.
-  const unsigned b = threadIdx.x & 255;
-  const float hi = __int_as_float(__builtin_amdgcn_ds_bpermute((int)((b >> 4) << 2), lut));
-  const float lo = __int_as_float(__builtin_amdgcn_ds_bpermute((int)((b & 15) << 2), lut));
-  const float2 e = make_float2(hi, lo);
-  // with 512 threads the second 256 fill the other half of the columns
-  const int j0 = threadIdx.x < 256 ? 0 : 16;
-  const int nj = blockDim.x > 256 ? 16 : 32;
-  for (int j = 0; j < nj; ++j) tab[b * 32 + ((j0 + j + b) & 31)] = e;
-}
-
-// Codebook value c (0..15) from immediate constants (a select chain): no
-// memory load, so a table built from it need not wait for any.
-__device__ __forceinline__ float nf4_code_imm(unsigned c) {
-  float r = -1.0f;
-  r = c == 1 ? -0.6961928009986877f : r;
-  r = c == 2 ? -0.5250730514526367f : r;
-  r = c == 3 ? -0.39491748809814453f : r;
-  r = c == 4 ? -0.28444138169288635f : r;
-  r = c == 5 ? -0.18477343022823334f : r;
-  r = c == 6 ? -0.09105003625154495f : r;
-  r = c == 7 ? 0.0f : r;
-  r = c == 8 ? 0.07958029955625534f : r;
-  r = c == 9 ? 0.16093020141124725f : r;
-  r = c == 10 ? 0.24611230194568634f : r;
-  r = c == 11 ? 0.33791524171829224f : r;
-  r = c == 12 ? 0.44070982933044434f : r;
-  r = c == 13 ? 0.5626170039176941f : r;
-  r = c == 14 ? 0.7229568362236023f : r;
-  r = c == 15 ? 1.0f : r;
-  return r;
-}
-
-// The pair table of init_pair_table (64 KiB at LDS offset 0, 32 lane
-// columns) filled by 512 threads from nf4_code_imm: thread t fills 16
-// columns of byte t % 256.
-__device__ __forceinline__ void init_pair_table_imm(char* smem) {
-  const unsigned b = threadIdx.x & 255;
-  const float2 e = make_float2(nf4_code_imm(b >> 4), nf4_code_imm(b & 15));
-  const int j0 = threadIdx.x < 256 ? 0 : 16;
-  float2* tab = reinterpret_cast<float2*>(smem);
-#pragma unroll
-  for (int j = 0; j < 16; ++j) tab[b * 32 + ((j0 + j + b) & 31)] = e;
-}
-
-__device__ __forceinline__ unsigned bf16x2_bits(float lo, float hi) {
-  bf16x2_t r = {(__bf16)lo, (__bf16)hi};  // v_cvt_pk_bf16_f32, RNE
-  return __builtin_bit_cast(unsigned, r);
-}
-
-// 8 NF4 elements of one packed dword -> 4 dwords of bf16 pairs in k order.
-// lane_off = (lane % 32) * 8: the lane's private column in the pair table.
-__device__ __forceinline__ u32x4_t nf4_dword_to_bf16(const float2* tab, unsigned x,
-                                                     unsigned lane_off, float s) {
-  u32x4_t r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned addr = __builtin_amdgcn_perm(x, lane_off, 0x0C0C0000u | ((4u + i) << 8));
-    const float2 p = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tab) + addr);
-    r[i] = bf16x2_bits(p.x * s, p.y * s);
-  }
-  return r;
-}
-
-// Same, with the table at an LDS address below 16 MiB whose bits 8..15 are
-// zero: `base_lane` = table address | lane column, and the address of byte b
-// is base_lane with b in bits 8..15 (one v_perm_b32). `lds0` points at LDS
-// address 0.
-__device__ __forceinline__ u32x4_t nf4_dword_to_bf16_at(const char* lds0, unsigned x,
-                                                        unsigned base_lane, float s) {
-  u32x4_t r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned addr = __builtin_amdgcn_perm(x, base_lane, 0x0C020000u | ((4u + i) << 8));
-    const float2 p = *reinterpret_cast<const float2*>(lds0 + addr);
-    r[i] = bf16x2_bits(p.x * s, p.y * s);
-  }
-  return r;
-}
-
-// ---- exact three-part NF4 codebook (decode kernels) ----
-//
-// Every fp32 codebook value v splits exactly into three bf16 values,
-// v = hi + mid + lo: hi keeps the top 16 bits of v's pattern (sign, exponent,
-// 7 mantissa bits), the remainder r = v - hi is exact with at most 16
-// significant bits, mid keeps r's top 16 bits and lo = r - mid is exact with
-// at most 8 significant bits. Three bf16 MFMAs over the parts therefore sum
-// codebook values at full fp32 precision (each product of a bf16 activation
-// and a bf16 part is exact in fp32), and absmax multiplies the 64-element
-// block sum once, in fp32, as the reference's GEMV does
-// (kernel/nf4_grouped.py:508-511).
-//
-// The split table: 256 bytes x 16 lane columns x 16 B = 64 KiB. Entry (byte,
-// column) holds the bf16 pairs (part[byte >> 4], part[byte & 15]) of hi, mid
-// and lo in dwords 0..2 (element 2j, the high nibble, in the low half), so
-// one 16-byte LDS read decodes a byte into the three MFMA operand dwords.
-// Column = lane % 16: the 16 lanes of one LDS pass read distinct banks.
-constexpr int kSplitCols = 16;
-constexpr int kSplitTabBytes = 256 * kSplitCols * 16;
-static_assert(kSplitTabBytes == 8 * kPairEntries, "split and pair tables take the same LDS");
-
-__device__ __forceinline__ void nf4_split_parts(int lut, unsigned& himid, unsigned& lo) {
-  const unsigned u = (unsigned)lut;
-  const unsigned h = u & 0xFFFF0000u;
-  const float r = __uint_as_float(u) - __uint_as_float(h);          // exact
-  const unsigned rm = __float_as_uint(r) & 0xFFFF0000u;
-  const float l = r - __uint_as_float(rm);                           // exact
-  himid = (h >> 16) | rm;                  // hi in the low half, mid in the high half
-  lo = __float_as_uint(l) >> 16;
-}
-
-// Fill the split table from the codebook register of lanes 0..15 (see
-// nf4_lut_lane). Thread t fills byte t % 256; with 512 threads each byte's
-// 16 columns are split over two threads. Columns rotate with the byte so one
-// store instruction touches distinct banks.
-__device__ __forceinline__ void init_split_table(char* tab, int lut) {
-  unsigned hm, lo;
-  nf4_split_parts(lut, hm, lo);
-  const unsigned b = threadIdx.x & 255;
-  const unsigned hmh = __builtin_amdgcn_ds_bpermute((int)((b >> 4) << 2), (int)hm);
-  const unsigned hml = __builtin_amdgcn_ds_bpermute((int)((b & 15) << 2), (int)hm);
-  const unsigned loh = __builtin_amdgcn_ds_bpermute((int)((b >> 4) << 2), (int)lo);
-  const unsigned lol = __builtin_amdgcn_ds_bpermute((int)((b & 15) << 2), (int)lo);
-  const u32x4_t e = {(hmh & 0xFFFFu) | (hml << 16), (hmh >> 16) | (hml & 0xFFFF0000u),
-                     loh | (lol << 16), 0u};
-  const int nj = blockDim.x > 256 ? 8 : 16;
-  const int j0 = threadIdx.x < 256 ? 0 : 8;
-  for (int j = 0; j < nj; ++j)
-    *reinterpret_cast<u32x4_t*>(tab + b * (kSplitCols * 16) + (((j0 + j + b) & 15) * 16)) = e;
-}
-
-// 16-byte LDS read at a byte address: no base pointer arithmetic around it.
-typedef __attribute__((address_space(3))) const u32x4_t lds_u32x4_t;
-__device__ __forceinline__ u32x4_t lds_read16(unsigned addr) {
-  return *(lds_u32x4_t*)(size_t)addr;
-}
-// The three bf16 parts of the four bytes of w (lane column lane_off), as the
-// hi, mid and lo MFMA operands. One 16-byte read per byte: three separate
-// 4-byte reads per byte into the operand registers measured 1.85x slower
-// (three times the LDS instructions, four lanes per bank), 12-byte reads
-// 2-10 % slower.
-__device__ __forceinline__ void split_lookup(unsigned w, unsigned lane_off, u32x4_t& hi,
-                                             u32x4_t& mid, u32x4_t& lo) {
-  u32x4_t d[4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-    d[b] = lds_read16(__builtin_amdgcn_perm(w, lane_off, 0x0C0C0000u | ((4u + b) << 8)));
-  hi = u32x4_t{d[0][0], d[1][0], d[2][0], d[3][0]};
-  mid = u32x4_t{d[0][1], d[1][1], d[2][1], d[3][1]};
-  lo = u32x4_t{d[0][2], d[1][2], d[2][2], d[3][2]};
-}
-typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-typedef __attribute__((address_space(3))) const f32x2_t lds_f32x2_t;
-__device__ __forceinline__ f32x2_t lds_read8f(unsigned addr) {
-  return *(lds_f32x2_t*)(size_t)addr;
-}
-
-// 8 MXFP4 elements of one packed dword (low nibble first) -> 4 bf16 pairs.
-__device__ __forceinline__ u32x4_t mx_dword_to_bf16(unsigned x, float s) {
-  u32x4_t r;
-  r[0] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, s, 0));
-  r[1] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, s, 1));
-  r[2] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, s, 2));
-  r[3] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, s, 3));
-  return r;
-}
-
-// e8m0 byte -> fp32 2^(e - 127): e = 0 is the subnormal 2^-127, e = 255 is
-// +inf (so a 0xFF block decodes to +-inf, and zero codes to NaN, like an
-// exp2-multiply decode; reference kernel/mxfp4_grouped.py:13-15).
-__device__ __forceinline__ float e8m0_to_f32(unsigned e) {
-  return __uint_as_float(e == 0 ? 0x00400000u : (e << 23));
-}
-
-// Calls fn(integral_constant<I>) for I = 0 .. S - 1 while it returns true.
-template <int I, int S>
-struct StepUnroll {
-  template <class Fn>
-  __device__ __forceinline__ static bool run(Fn& fn) {
-    if (!fn(std::integral_constant<int, I>{})) return false;
-    return StepUnroll<I + 1, S>::run(fn);
-  }
-};
-template <int S>
-struct StepUnroll<S, S> {
-  template <class Fn>
-  __device__ __forceinline__ static bool run(Fn&) { return true; }
-};
-
-__device__ __forceinline__ bf16x8_t as_bf16x8(u32x4_t v) {
-  return __builtin_bit_cast(bf16x8_t, v);
-}
-
-__device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
-}
-
-// Activation chunk (8 consecutive elements) as bf16 bits. fp16 inputs are
-// rejected on the host before launch; the kernels take bf16.
-__device__ __forceinline__ u32x4_t load_a8(const uint16_t* p) {
-  return *reinterpret_cast<const u32x4_t*>(p);
-}
-
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  __bf16 b = (__bf16)f;
-  return __builtin_bit_cast(uint16_t, b);
-}
-
-// ============================================================ decode fwd ==
-
-struct FwdArgs {
-  const uint16_t* a;        // [T, lda] bf16
-  int64_t lda;
-  const uint8_t* B;         // [E, N, K/2]
-  int64_t sbe, sbn;         // bytes
-  const void* S;            // absmax f32 [E, N, K/64] or e8m0 u8 [E, N, K/32]
-  int64_t sse, ssn;         // elements
-  const int32_t* eids;      // [G]
-  const int32_t* row_off;   // [G + 1] (ro_shift 0), [2 G] (ro_shift 1), or
-                            // null: group g is the single row g
-  const int32_t* t_row0;    // [n_mtiles] (gemm path)
-  const int32_t* t_rows;
-  const int32_t* t_group;
-  int n_mtiles;
-  int G;
-  int max_m;                // largest group (decode path)
-  // decode path: group g's rows are [row_off[g << ro_shift],
-  // row_off[(g << ro_shift) + 1]): ro_shift 0 reads the G + 1 prefix offsets,
-  // 1 a (first, end) pair per group, so the groups may come in any order
-  int ro_shift;
-  int64_t N, K;
-  uint16_t* out;            // [T, ldo] bf16
-  int64_t ldo;
-  // host only: group ids and row offsets to pass in the GEMV kernels'
-  // arguments (GemvIds), or null (the kernels read eids / row_off)
-  const struct GemvIds* ids_inline;
-  // host only: the groups come from device routing and any of them may be
-  // empty (the launch covers a bound of the active groups)
-  int sparse_groups;
-};
-
-// The groups of a decode launch of at most kGemvIdsMax groups, in the GEMV
-// kernels' arguments (n > 0): the kernel reads them from the kernarg
-// segment it loads anyway, instead of a table in memory behind it (one
-// dependent round trip before the first weight load). Entry y (grid row y)
-// is a group: its expert id e[y] and rows[y] = first row << 8 | row count.
-// The host lists the groups largest first, so the workgroups of the groups
-// that take the most passes are dispatched first (every output row is
-// computed on its own: the order changes no bits). has_ro: the caller gave
-// row offsets (the multi-row GEMV needs them).
-constexpr int kGemvIdsMax = 384;
-constexpr int kGemvRowsMax = 1 << 23;   // first rows must fit in rows[y] >> 8
-struct GemvIds {
-  int32_t e[kGemvIdsMax];
-  int32_t rows[kGemvIdsMax];
-  int32_t n;
-  int32_t has_ro;
-};
-
-constexpr int kOOB = (int)0x80000000;  // buffer offset past every resource: loads 0
-
-// Buffer resources: raw loads through them are bounds-checked by the
-// hardware, so a masked lane gets zeros without a branch (and the compiler
-// keeps exact vmcnt counts for the prefetched loads).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int64_t bytes) {
-  const int n = bytes < 0x7FFFFFFF ? (int)bytes : 0x7FFFFFFF;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, 0x00020000);
-}
-
-__device__ __forceinline__ u32x4_t buf_load16(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-
-// Cache-policy bits of a buffer access: kScopeDevice (sc1) makes the access
-// coherent at device scope, across the XCDs' separate L2 caches, without any
-// cache writeback or invalidate.
-constexpr int kScopeDevice = 16;
-
-template <int kAux>
-__device__ __forceinline__ u32x4_t buf_load16_aux(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kAux));
-}
-
-__device__ __forceinline__ unsigned buf_load1(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, 0);
-}
-
-// off | 0x80000000 when !ok, through an opaque VALU op so the compiler cannot
-// turn the masked load back into a branch around two loads.
-__device__ __forceinline__ int oob_unless(bool ok, int off) {
-  const int mask = ok ? 0 : kOOB;
-  int r;
-  asm volatile("v_or_b32 %0, %1, %2" : "=v"(r) : "v"(off), "v"(mask));
-  return r;
-}
-
-template <int FMT>
-__device__ __forceinline__ float load_scale(const FwdArgs& p, int64_t e, int64_t n, int64_t k) {
-  if constexpr (FMT == kNF4) {
-    const float* s = static_cast<const float*>(p.S);
-    return s[e * p.sse + n * p.ssn + (k >> 6)];
-  } else {
-    const uint8_t* s = static_cast<const uint8_t*>(p.S);
-    return e8m0_to_f32(s[e * p.sse + n * p.ssn + (k >> 5)]);
-  }
-}
 
 // Unit kinds of the decode body.
 //   kPlain   out = a . W^T over the unit's 16 * kTiles rows.
@@ -2297,357 +1954,17 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm_fwd(const FwdArgs p) {
   }
 }
 
-// ============================================================== prefill ==
-//
-// Tiled forward for groups larger than the decode path takes. Tile: 128 rows
-// of one group x 256 weight rows (n); four waves, wave w owns the 64 weight
-// rows [64 w, 64 w + 64) for all 128 activation rows, so no weight element is
-// decoded twice. K advances in steps of 64.
-//
-//   * weights: each lane loads 8 packed bytes (16 k values) per 16-row
-//     n-subtile and step straight into registers and decodes them into two
-//     MFMA operands (the weights are MFMA operand A, so the accumulator holds
-//     out^T and a lane ends with 4 consecutive output columns of one row);
-//   * activations: a ring of three 16 KiB LDS stages filled by buffer loads
-//     that write LDS directly (no VGPR round trip). A stage holds 128 rows x
-//     64 k; 16-byte slots are swizzled per row (pf_swz) so the 16-byte
-//     operand reads of a wave run at the full 256 B per clock;
-//   * one flat software pipeline over (tile, k-step) pairs of the workgroup's
-//     whole tile list: the loads of step f + 2 are in flight while step f
-//     computes, across tile boundaries;
-//   * tiles: a persistent grid; the tile list (m-tile major, n-tile minor, so
-//     a group's tiles are adjacent) is cut into eight contiguous ranges, one
-//     per XCD (workgroup b runs on XCD b % 8), so the tiles an XCD runs at
-//     the same time share weights and activations in that XCD's L2.
-//
-// Every vector-memory instruction of a step is counted: kPfGroupLoads per
-// step and wave. The waits on the LDS stages are explicit s_waitcnt
-// immediates computed from that count (stores only add to the count, which
-// makes a wait stricter, never looser).
+// ================================================= tiles: shared constants ==
+
 constexpr int kPfBM = 128;
 constexpr int kPfBN = 256;
 constexpr int kPfBK = 64;
 constexpr int kPfStage = kPfBM * kPfBK * 2; // bytes per LDS stage
 
-// s_waitcnt with vmcnt(n) and lgkmcnt(0), expcnt untouched (gfx9 encoding).
-template <int n>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-  static_assert(n >= 0 && n < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14));
-}
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// Values the kernel knows to be wave-uniform but the compiler may not (it
-// would otherwise keep buffer descriptors in VGPRs and loop over lanes).
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <class T>
-__device__ __forceinline__ void* uniform_ptr(const T* ptr) {
-  const uint64_t v = reinterpret_cast<uint64_t>(ptr);
-  const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-  const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-  return reinterpret_cast<void*>(lo | (hi << 32));
-}
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-// LDS slot swizzle of a staged activation row: 16-byte slot s of row m lives
-// at slot s ^ pf_swz(m % 16). Over the 16 rows one operand read touches this
-// spreads the 16-byte pieces across all 64 banks.
-__device__ __forceinline__ int pf_swz(int m16) { return (m16 ^ (m16 >> 3)) & 7; }
-
-struct PfTile {
-  int row0, rows, e, n0;
-};
-
-
-template <int FMT, int kS>
-__global__ void __launch_bounds__(512, 2)
-    k_prefill(const FwdArgs p, const int32_t* __restrict__ t_row0,
-              const int32_t* __restrict__ t_rows, const int32_t* __restrict__ t_group,
-              const int32_t* __restrict__ eids, uint16_t* __restrict__ out) {
-  static_assert(kS == 4, "ring depth: even, and four 16 KiB stages fill the low 64 KiB");
-  constexpr int kWaves = 8;
-  constexpr int kWaveCols = kPfBN / kWaves;          // 32: one 32 x 32 MFMA column block
-  constexpr int kAPieces = kPfStage / 1024 / kWaves; // LDS-direct loads per wave and step
-  constexpr int kRowsPerWave = kPfBM / kWaves;
-  constexpr int kGroupLoads = kAPieces + 2;          // + weights + scale
-  constexpr int kMT = kPfBM / 32;                    // activation subtiles of 32 rows
-  static_assert(kWaveCols == 32, "one weight subtile per wave");
-  // one LDS object per stage, so the compiler can tell the stages apart when
-  // it places the waits for the direct-to-LDS loads
-  __shared__ __attribute__((aligned(16))) char s_a0[kPfStage];
-  __shared__ __attribute__((aligned(16))) char s_a1[kPfStage];
-  __shared__ __attribute__((aligned(16))) char s_a2[kPfStage];
-  __shared__ __attribute__((aligned(16))) char s_a3[kPfStage];
-  // NF4 pair table: dynamic LDS, which follows the 64 KiB of static stages, so
-  // it starts at 0x10000 and the stages keep addresses an instruction's
-  // 16-bit offset field can hold.
-  extern __shared__ __attribute__((aligned(16))) float2 s_tab[];
-  auto stage_of = [&](auto RI) -> char* {
-    constexpr int r = decltype(RI)::value;
-    if constexpr (r == 0) return s_a0;
-    else if constexpr (r == 1) return s_a1;
-    else if constexpr (r == 2) return s_a2;
-    else return s_a3;
-  };
-  const int lut = FMT == kNF4 ? nf4_lut_lane() : 0;
-  __builtin_amdgcn_sched_barrier(0);
-  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-  const int l32 = lane & 31, h = lane >> 5;
-  // table base (0x10000: byte 2) | lane column; nf4_dword_to_bf16_at takes
-  // byte 2 of this register as address byte 2
-  const unsigned tab_base = (unsigned)(uintptr_t)s_tab;
-  const unsigned lane_off = tab_base | (unsigned)(lane & 31) * 8u;
-  const char* lds0 = reinterpret_cast<const char*>(s_tab) - tab_base;
-  constexpr int kScaleBytes = FMT == kNF4 ? 4 : 1;
-
-  // ---- this workgroup's tiles
-  const int n_tiles = (int)((p.N + kPfBN - 1) / kPfBN);
-  const int64_t total = (int64_t)p.n_mtiles * n_tiles;
-  const int nx = gridDim.x >= 8 ? 8 : 1;
-  const int x = (int)(blockIdx.x % nx), slot = (int)(blockIdx.x / nx);
-  const int wpx = (int)((gridDim.x - x + nx - 1) / nx);   // workgroups on this XCD
-  const int64_t lo = total * x / nx, hi = total * (x + 1) / nx;
-  const int my_tiles = lo + slot < hi ? (int)((hi - lo - slot + wpx - 1) / wpx) : 0;
-  const int ksteps = (int)((p.K + kPfBK - 1) / kPfBK);
-  const int F = my_tiles * ksteps;
-  if constexpr (FMT == kNF4) init_pair_table(s_tab, lut);
-  if (F == 0) return;
-
-  // Tile descriptors come in through scalar loads (counted by lgkmcnt, so
-  // they never disturb the vector-memory counts the stage waits rely on).
-  auto meta = [&](int j) {
-    PfTile t;
-    const int64_t tg = lo + slot + (int64_t)j * wpx;
-    const int mt = (int)(tg / n_tiles);
-    t.n0 = (int)(tg - (int64_t)mt * n_tiles) * kPfBN;
-    t.row0 = t_row0[mt];
-    t.rows = t_rows[mt];
-    t.e = eids[t_group[mt]];
-    return t;
-  };
-
-  // ---- per-lane constants
-  const int64_t lda2 = p.lda * 2;
-  // A stage: wave w fills its kRowsPerWave rows, 8 rows per instruction
-  int a_row[kAPieces], a_slot[kAPieces];
-#pragma unroll
-  for (int i = 0; i < kAPieces; ++i) {
-    a_row[i] = wave * kRowsPerWave + i * 8 + (lane >> 3);
-    a_slot[i] = (lane & 7) ^ pf_swz(a_row[i] & 15);
-  }
-  // MFMA k mapping within a 64-wide step: lane half h covers k [32 h, 32 h + 32),
-  // MFMA kk (0..3) takes k [32 h + 8 kk, +8) -- 16-byte slot 4 h + kk of a row.
-  // Activation operand kk of subtile i: row i * 32 + l32 at i * 4096 + a_off[kk].
-  int a_off[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) a_off[kk] = l32 * 128 + ((4 * h + kk) ^ pf_swz(l32 & 15)) * 16;
-
-  // ---- ring state
-  u32x4_t wreg[kS];      // 16 packed bytes: row n, k [k0 + 32 h, +32)
-  unsigned sreg[kS];     // its absmax (NF4) or e8m0 byte (MXFP4)
-  PfTile ring_t[kS];
-  bool ring_last[kS];
-  f32x16_t acc[kMT];
-#pragma unroll
-  for (int i = 0; i < kMT; ++i) acc[i] = f32x16_t{};
-
-  // ---- issue state: the tile the issue pointer is in. Per tile: buffer
-  // resources and per-lane offsets, with rows and columns outside the tile
-  // folded into out-of-range offsets; per step only the k offset (a scalar
-  // soffset) changes. Steps past the end use zero-size resources, so every
-  // step issues the same instructions and the vector-memory counts hold.
-  int iss_j = 0, iss_ks = 0;
-  PfTile iss_t;
-  const char* a_base = nullptr;
-  const uint8_t* b_base = nullptr;
-  const char* s_base = nullptr;
-  int a_bytes = 0, b_bytes = 0, s_bytes = 0;
-  int a_voff[kAPieces], b_voff = 0, s_voff = 0;
-  auto tile_setup = [&](int j) {
-    iss_t = meta(j);
-    a_base = reinterpret_cast<const char*>(p.a + (int64_t)iss_t.row0 * p.lda);
-    a_bytes = (int)((int64_t)iss_t.rows * lda2);
-#pragma unroll
-    for (int i = 0; i < kAPieces; ++i)
-      a_voff[i] = a_row[i] < iss_t.rows ? (int)(a_row[i] * lda2) + a_slot[i] * 16 : kOOB;
-    b_base = p.B + (int64_t)iss_t.e * p.sbe;
-    b_bytes = (int)(p.N * p.sbn);
-    s_base = static_cast<const char*>(p.S) + (int64_t)iss_t.e * p.sse * kScaleBytes;
-    s_bytes = (int)(p.N * p.ssn * kScaleBytes);
-    const int64_t n = iss_t.n0 + wave * kWaveCols + l32;
-    b_voff = n < p.N ? (int)(n * p.sbn) + h * 16 : kOOB;
-    if constexpr (FMT == kNF4) s_voff = n < p.N ? (int)(n * p.ssn * 4) : kOOB;
-    else s_voff = n < p.N ? (int)(n * p.ssn) + h : kOOB;
-  };
-  tile_setup(0);
-
-  auto issue = [&](auto RI, char* stage, bool live) {
-    constexpr int r = decltype(RI)::value;
-    const int k0 = uniform(iss_ks) * kPfBK;
-    live = uniform(live ? 1 : 0) != 0;
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-        uniform_ptr(a_base), 0, uniform(live ? a_bytes : 0), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-        uniform_ptr(b_base), 0, uniform(live ? b_bytes : 0), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        uniform_ptr(s_base), 0, uniform(live ? s_bytes : 0), 0x00020000);
-#pragma unroll
-    for (int i = 0; i < kAPieces; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ra, (lds_ptr_t)(stage + (wave * kAPieces + i) * 1024), 16, a_voff[i], k0 * 2, 0, 0);
-    wreg[r] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, b_voff, k0 >> 1, 0));
-    if constexpr (FMT == kNF4)
-      sreg[r] = __builtin_amdgcn_raw_buffer_load_b32(rs, s_voff, (k0 >> 6) * 4, 0);
-    else
-      sreg[r] = __builtin_amdgcn_raw_buffer_load_b8(rs, s_voff, k0 >> 5, 0);
-    ring_t[r] = iss_t;
-    ring_last[r] = iss_ks == ksteps - 1;
-    // advance
-    if (++iss_ks == ksteps) {
-      iss_ks = 0;
-      ++iss_j;
-      if (iss_j < my_tiles) tile_setup(iss_j);
-    }
-  };
-
-  // Decoded weight operands: wf[r % 2] holds step f's (ring slot r)
-  // operands, decoded during step f - 1 (kS is even, so the two buffers
-  // alternate without copies).
-  u32x4_t wf[2][4];
-  auto decode = [&](auto RI) {
-    constexpr int r = decltype(RI)::value;
-    if constexpr (FMT == kNF4) {
-      const float s = __uint_as_float(sreg[r]);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        wf[r & 1][kk] = nf4_dword_to_bf16_at(lds0, wreg[r][kk], lane_off, s);
-    } else {
-      const float s = e8m0_to_f32(sreg[r]);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) wf[r & 1][kk] = mx_dword_to_bf16(wreg[r][kk], s);
-    }
-  };
-
-  // MFMAs of step f (slot r) over the first kM activation subtiles. The
-  // weights are operand A, so acc[i] holds out^T: lane (l32, h) gets token
-  // row i * 32 + l32 and columns 8 g + 4 h + (0..3), g = 0..3.
-  auto mma = [&](auto RI, auto MI, const char* stage, auto&& after_first) {
-    constexpr int r = decltype(RI)::value;
-    constexpr int kM = decltype(MI)::value;
-    // operands of k-slices kk and kk + 1 in flight; the reads for kk + 2 go
-    // out right after kk's MFMAs, so each MFMA's operand has had a full
-    // k-slice of MFMAs to arrive
-    u32x4_t av[2][kM];
-    auto read = [&](int buf, int kk) {
-#pragma unroll
-      for (int i = 0; i < kM; ++i)
-        av[buf][i] = *reinterpret_cast<const u32x4_t*>(stage + a_off[kk] + i * 4096);
-    };
-    read(0, 0);
-    read(1, 1);
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < kM; ++i)
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wf[r & 1][kk]),
-                                                          as_bf16x8(av[kk & 1][i]), acc[i], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (kk == 0) {
-        after_first();
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (kk + 2 < 4) read(kk & 1, kk + 2);
-    }
-  };
-
-  // The two waves that share a SIMD (w and w + 4) run the step's two halves
-  // in opposite orders -- decode of step f + 1 then MFMAs of step f, or the
-  // reverse -- so while one wave decodes on the VALU the other keeps the
-  // matrix core busy. The order is a template argument of the whole loop
-  // (each wave half runs its own copy), so no step merges two orders.
-  auto mma_decode = [&](auto RI, auto MI, auto DF, const char* stage, auto&& after_first) {
-    constexpr int r = decltype(RI)::value;
-    if constexpr (decltype(DF)::value) {
-      decode(std::integral_constant<int, (r + 1) % kS>{});
-      __builtin_amdgcn_sched_barrier(0);
-      mma(RI, MI, stage, after_first);
-    } else {
-      mma(RI, MI, stage, after_first);
-      __builtin_amdgcn_sched_barrier(0);
-      decode(std::integral_constant<int, (r + 1) % kS>{});
-    }
-  };
-
-  auto compute = [&](auto RI, auto DF, const char* stage, auto&& after_first) {
-    constexpr int r = decltype(RI)::value;
-    const int rows = uniform(ring_t[r].rows);
-    // every tile runs all 4 subtiles (rows past the group are zeros in LDS):
-    // one straight-line step keeps the accumulators in place
-    mma_decode(RI, std::integral_constant<int, 4>{}, DF, stage, after_first);
-    if (ring_last[r]) {
-      const PfTile t = ring_t[r];
-      const int n_l = t.n0 + wave * kWaveCols + 4 * h;   // lane's first column
-      uint16_t* o = out + (int64_t)(t.row0 + l32) * p.ldo + n_l;
-#pragma unroll
-      for (int i = 0; i < kMT; ++i) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if (i * 32 + l32 < rows && n_l + 8 * g < p.N) {
-            uint2 v;
-            v.x = bf16x2_bits(acc[i][4 * g + 0], acc[i][4 * g + 1]);
-            v.y = bf16x2_bits(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-            *reinterpret_cast<uint2*>(o + (int64_t)i * 32 * p.ldo + 8 * g) = v;
-          }
-        }
-        acc[i] = f32x16_t{};
-      }
-    }
-  };
-
-  // Step f: wait for stage f (loads issued after it: the kS - 2 younger
-  // stages), barrier, compute; the refill of the stage read in step f - 1
-  // with step f + kS - 1 goes out after the first k-slice's MFMAs, so the
-  // eight waves' loads do not queue up behind the barrier all at once.
-  int f = 0;
-  auto step = [&](auto RI, auto DF) {
-    constexpr int r = decltype(RI)::value;
-    constexpr int rf = (r + kS - 1) % kS;
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vm_lgkm0<(kS - 2) * kGroupLoads>();
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    const bool live = f + kS - 1 < F;
-    compute(RI, DF, stage_of(RI), [&]() {
-      issue(std::integral_constant<int, rf>{}, stage_of(std::integral_constant<int, rf>{}), live);
-    });
-    return ++f < F;
-  };
-
-  issue(std::integral_constant<int, 0>{}, s_a0, true);
-  issue(std::integral_constant<int, 1>{}, s_a1, F > 1);
-  if constexpr (kS > 3) issue(std::integral_constant<int, 2>{}, s_a2, F > 2);
-  if constexpr (FMT == kNF4) __syncthreads();  // pair table complete
-  decode(std::integral_constant<int, 0>{});
-  if (wave < kWaves / 2) {
-    auto st = [&](auto RI) { return step(RI, std::true_type{}); };
-    while (StepUnroll<0, kS>::run(st)) {
-    }
-  } else {
-    auto st = [&](auto RI) { return step(RI, std::false_type{}); };
-    while (StepUnroll<0, kS>::run(st)) {
-    }
-  }
-  // the past-the-end direct-to-LDS loads (zero-size resources) still write
-  // their LDS slots: let them land before the workgroup's LDS is released
-  __builtin_amdgcn_s_waitcnt(0);
-}
 
 // 256-row tiles (k_prefill_w below).
 constexpr int kPtBM = 256;
-// cache-policy operand of a buffer store: nt (non-temporal) on gfx950
-constexpr int kNonTemporal = 2;
 constexpr int kPtStage = kPtBM * kPfBK * 2;
 
 // Pair table with 16 columns: entry (byte b, column c) at b * 128 + c * 8.
@@ -3200,19 +2517,6 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   }
 }
 
-// A tile table small enough to travel in the kernel arguments (n > 0): no
-// upload, so a call needs no copy ahead of its launch (and a captured graph
-// no copy node). grp holds the group index, or the expert id itself where
-// the caller knows the ids on the host (grp_is_expert). 3 KiB, inside the
-// kernel-argument limit with FwdArgs.
-constexpr int kPwMaxTiles = 256;
-struct PwTiles {
-  int32_t row0[kPwMaxTiles];
-  int32_t rows[kPwMaxTiles];
-  int32_t grp[kPwMaxTiles];
-  int32_t n;
-  int32_t grp_is_expert;
-};
 
 template <int FMT, bool DG = false>
 __global__ void __launch_bounds__(256, 1)
@@ -4377,7 +3681,7 @@ const PwTiles& no_tiles() {
   return empty;
 }
 
-// Workgroups per XCD range of the persistent k_prefill_w grid: one per CU
+// Workgroups per XCD range of the persistent tile grids: one per CU
 // (each walks several tiles; the pair table is built once per workgroup), or
 // fewer when the XCD's range has fewer tiles.
 int64_t prefill_w_per_xcd(int64_t tiles, int cus) {
@@ -4394,40 +3698,21 @@ int launch_fwd(const FwdArgs& p, int block_m, hipStream_t stream, const PwTiles*
     const int rc = launch_decode<FMT>(p, stream);
     if (rc) return rc;
   } else {
-    const bool pf_ok = p.N % 4 == 0 && p.ldo % 4 == 0 && p.K % kPfBK == 0 &&
-                       (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM &&
-                       (int64_t)kPtBM * p.lda * 2 < 0x7FFFFFFF;
-    if (tt && block_m != kPtBM) return -1;   // kernel-argument tables: four-wave kernel only
-    if (block_m == kPtBM) {
-      // 256-row tiles: the host picks them only where the four-wave kernel
-      // takes the shape
-      if (!pf_ok || (int64_t)kPtBM * p.ldo * 2 >= 0x7FFFFFFF) return -1;
+    // k_tile_fwd: tables of any height up to 256 rows (each row is computed
+    // the same way in every tile), whole 64-wide k steps, 4-column stores
+    const bool tile_ok = p.N % 4 == 0 && p.ldo % 4 == 0 && p.K % kPfBK == 0 &&
+                         (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM &&
+                         (int64_t)kPtBM * p.lda * 2 < 0x7FFFFFFF &&
+                         (int64_t)kPtBM * p.ldo * 2 < 0x7FFFFFFF;
+    if (tile_ok) {
       const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kPfBN - 1) / kPfBN);
       // the grid covers eight equal XCD ranges
       const int64_t per_x = prefill_w_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
-      hipLaunchKernelGGL((k_prefill_w<FMT>), dim3((unsigned)(per_x * 8)), dim3(256), 0, stream, p,
-                         p.t_row0, p.t_rows, p.t_group, p.eids, p.out, tt ? *tt : no_tiles());
-      return hipGetLastError() == hipSuccess ? 0 : -2;
+      return launch_tile_fwd(FMT, p, tt ? *tt : no_tiles(), per_x, stream);
     }
-    if (block_m > kPfBM) return -1;
-    if (pf_ok) {
-      const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kPfBN - 1) / kPfBN);
-      int64_t grid = tiles < cus ? tiles : cus;
-      const int dyn = FMT == kNF4 ? 8 * kPairEntries : 0;
-      static int configured_dev = -1;
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess) return -2;
-      if (dyn && configured_dev != dev) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_prefill<FMT, 4>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, dyn) != hipSuccess)
-          return -2;
-        configured_dev = dev;
-      }
-      hipLaunchKernelGGL((k_prefill<FMT, 4>), dim3((unsigned)grid), dim3(512), dyn, stream, p,
-                         p.t_row0, p.t_rows, p.t_group, p.eids, p.out);
-      return hipGetLastError() == hipSuccess ? 0 : -2;
-    }
+    // kernel-argument tables and 256-row tables are for that kernel only
+    if (tt || block_m > kPfBM) return -1;
     const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kBN - 1) / kBN);
     const int64_t grid = clamp_grid(tiles, cus);
     switch (block_m) {

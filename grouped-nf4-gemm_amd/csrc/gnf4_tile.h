@@ -1,0 +1,13 @@
+// gnf4_tile.h -- launches of the tile kernels (gnf4_tile.hip).
+#pragma once
+
+#include "gnf4_device.h"
+
+namespace gnf4 {
+
+// 256-row forward tiles on a grid of eight XCD ranges of per_x workgroups.
+// The tile table is tt's (n > 0) or p's device arrays.
+int launch_tile_fwd(int fmt, const FwdArgs& p, const PwTiles& tt, int64_t per_x,
+                    hipStream_t stream);
+
+}  // namespace gnf4

@@ -549,37 +549,27 @@ def _kernel_block_m(block_m: int) -> int:
     return 128
 
 
-def _auto_block_m(max_rows: int, K: int = 0) -> int:
-    """Tile height the forward uses when the caller names none: the
-    reference's group-size rule (``_prefill_block_m``), except that groups of
-    more than 128 rows, and any tiled call with K >= 1024, take the 256-row
-    tiles of the four-wave kernel (each decoded weight feeds up to twice the
-    rows; its tile prologue is paid back over a long K; the bits are the
-    same). Measured, 128 experts, Qwen3 shapes: K = 2048 runs 5-11 % faster
-    on 256-row tiles at 24-128 rows per group, K = 768 0-4 % slower at
-    100-128 rows."""
-    if max_rows > 128 or K >= 1024:
-        return 256
-    return _kernel_block_m(_prefill_block_m(max_rows))
-
-
 def _tall_tiles_ok(N: int, K: int) -> bool:
-    """Whether the library takes 256-row forward tiles for this shape (whole
-    64-wide k steps, 4-column output stores)."""
+    """Whether the library's tile kernel takes this shape (whole 64-wide k
+    steps, 4-column output stores), and with it tiles of up to 256 rows."""
     return K % 64 == 0 and N % 4 == 0
 
 
 def _fwd_block_m(max_m: int, N: int, K: int, block_m=None) -> int:
     """Tile height of a tiled forward launch, shared by the op and by
-    ``GroupPlan``: the caller's ``block_m`` rounded up to a supported
-    height, else ``_auto_block_m`` where the shape takes 256-row tiles, else
-    the reference's group-size rule."""
+    ``GroupPlan``: the caller's ``block_m`` rounded up to a supported height,
+    else 256 rows wherever the shape takes them (a tile computes only its
+    group's 32-row subtiles, and each decoded weight feeds all of them), else
+    the reference's group-size rule. Against 128-row tiles with every subtile
+    computed (MI355X): 128 experts, N = 2048, K = 768, 32 / 64 / 128 rows per
+    group 47.9 / 56.0 / 72.0 us against 61.0 / 68.5 / 88.1; 64 experts, N =
+    2048, K = 256, 32 / 128 rows 15.4 / 21.8 against 18.6 / 29.8; MXFP4, K =
+    512, 14.8 / 26.3 against 23.2 / 36.6."""
     if block_m is not None:
         return _kernel_block_m(block_m)
-    bm = _auto_block_m(max_m, K)
-    if bm == 256 and not _tall_tiles_ok(N, K):
-        bm = _kernel_block_m(_prefill_block_m(max_m))
-    return bm
+    if _tall_tiles_ok(N, K):
+        return 256
+    return _kernel_block_m(_prefill_block_m(max_m))
 
 
 # ------------------------------------------------------------------ launch --
