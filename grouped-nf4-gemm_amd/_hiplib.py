@@ -12,7 +12,7 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "libgnf4_hip.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 FMT_NF4 = 0
 FMT_MXFP4 = 1
@@ -23,6 +23,7 @@ DTYPE_F32 = 2
 _P = ctypes.c_void_p
 _I = ctypes.c_int
 _I64 = ctypes.c_int64
+_F = ctypes.c_float
 
 # name -> argtypes; every entry point returns int
 SIGNATURES = {
@@ -74,6 +75,10 @@ SIGNATURES = {
                            _P, _P, _P, _P, _I, _I, _I64, _I64, _P, _I64, _P],
     "gnf4_hip_mxfp4_dgrad": [_P, _I, _I64, _P, _I64, _I64, _P, _I64, _I64,
                              _P, _P, _P, _P, _I, _I, _I64, _I64, _P, _I64, _P],
+    "gnf4_hip_lora_down": [_P, _I64, _P, _I, _I64, _I64, _I, _P, _P, _P, _I, _I, _F, _P, _P],
+    "gnf4_hip_lora_up": [_P, _P, _I, _I64, _I64, _I, _P, _P, _P, _I, _I, _F, _P, _I64, _P, _I64,
+                         _P],
+    "gnf4_hip_lora_wgrad": [_P, _I64, _P, _I, _I64, _I64, _I, _P, _P, _I, _F, _P, _P],
 }
 
 # entry points that do not return int

@@ -1,7 +1,7 @@
 """Build libgnf4_hip.so in-tree for gfx950 with hipcc.
 
 ``python build.py`` (or ``build()``) compiles the HIP sources in csrc/ (the
-grouped GEMM kernels, its tile kernels and the routing kernels) into ``libgnf4_hip.so`` next to
+grouped GEMM kernels, its tile kernels, the routing and the LoRA kernels) into ``libgnf4_hip.so`` next to
 this file, and the measurement kernels bench.py times against
 (``csrc/gnf4_floor.hip``) into ``libgnf4_floor.so``. It always recompiles: the library must
 track its source, and the GPU box only ever loads the prebuilt file.
@@ -16,7 +16,8 @@ from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
-SRCS = [HERE / "csrc" / n for n in ("gnf4_hip.hip", "gnf4_tile.hip", "gnf4_route.hip")]
+SRCS = [HERE / "csrc" / n for n in ("gnf4_hip.hip", "gnf4_tile.hip",
+                                         "gnf4_route.hip", "gnf4_lora.hip")]
 OUT = HERE / "libgnf4_hip.so"
 FLOOR_SRCS = [HERE / "csrc" / "gnf4_floor.hip"]
 FLOOR_OUT = HERE / "libgnf4_floor.so"

@@ -14,8 +14,10 @@ Interface and semantics follow the reference's kernel/nf4_qlora.py:32-305
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
+import _hiplib
 import mxfp4_grouped
 import nf4_grouped
 
@@ -197,6 +199,129 @@ def _lora_delta_grouped_loop(a_cat, lora_A, lora_B, sizes, expert_ids, scaling=1
     return out
 
 
+# ------------------------------------------------- the fused low-rank kernels --
+
+def _transforming() -> bool:
+    """Whether something other than plain eager autograd watches the torch
+    calls (tracing, functorch transforms, forward-mode, dispatch or function
+    modes, autocast): then the torch composition runs, which they all see."""
+    from torch.autograd import forward_ad
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0
+            or torch.is_autocast_enabled())
+
+
+def _kernels_take(out, a_cat, lora_A, lora_B, sizes) -> bool:
+    """Whether the HIP kernels take this low-rank delta: bf16 rows and fp32
+    adapters on one GPU, plain contiguous tensors, r % 4 == 0 and r <= 64,
+    widths that are multiples of 8, every row in a group."""
+    ts = (out, a_cat, lora_A, lora_B)
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+               and t.device == out.device for t in ts):
+        return False
+    if (out.dtype, a_cat.dtype) != (torch.bfloat16, torch.bfloat16) or lora_A.dim() != 3:
+        return False
+    if (lora_A.dtype, lora_B.dtype) != (torch.float32, torch.float32) or lora_B.dim() != 3:
+        return False
+    (T, N), K = out.shape, a_cat.shape[1]
+    E, r, _ = lora_A.shape
+    return (tuple(lora_A.shape) == (E, r, K) and tuple(lora_B.shape) == (E, N, r)
+            and 0 < E <= 65535 and 4 <= r <= 64 and r % 4 == 0 and K % 8 == 0 and N % 8 == 0
+            and lora_A.is_contiguous() and lora_B.is_contiguous()
+            and lora_A.data_ptr() % 16 == 0 and lora_B.data_ptr() % 16 == 0
+            and T > 0 and sum(int(m) for m in sizes) == T and not _transforming())
+
+
+class _LoraTables:
+    """Device tables of one routing: tile and row offsets, expert ids."""
+
+    def __init__(self, sizes, expert_ids, dev):
+        m = np.asarray([int(v) for v in sizes], dtype=np.int32)
+        off = np.zeros((2, len(m) + 1), dtype=np.int32)
+        np.cumsum((m + 15) // 16, out=off[0, 1:])
+        np.cumsum(m, out=off[1, 1:])
+        ids = nf4_grouped._eids_device(expert_ids, dev)
+        host = [*off] + ([] if ids is not None else [nf4_grouped._np_ids(expert_ids)])
+        views = nf4_grouped.to_device_i32(host, dev)
+        self.n, self.G = int(off[0, -1]), len(m)
+        self.tile_off, self.row_off = views[:2]
+        self.ids = ids.contiguous() if ids is not None else views[2]
+
+    def args(self):
+        return (self.tile_off.data_ptr(), self.row_off.data_ptr(), self.ids.data_ptr(), self.G,
+                self.n)
+
+
+def _lora_call(name, dev, *args):
+    with nf4_grouped._device_ctx(dev):
+        rc = getattr(_hiplib.load(), name)(*args, nf4_grouped._stream_ptr(dev))
+    _hiplib.check(rc, "fused_grouped_lora")
+
+
+def _lora_down(x, w, transposed, tb, scale, r):
+    E, C = w.shape[0], x.shape[1]
+    y = torch.empty(x.shape[0], r, dtype=torch.float32, device=x.device)
+    _lora_call("gnf4_hip_lora_down", x.device, x.data_ptr(), x.stride(0), w.data_ptr(),
+               transposed, E, C, r, *tb.args(), scale, y.data_ptr())
+    return y
+
+
+def _lora_up(u, w, transposed, C, tb, scale, base=None):
+    T, r = u.shape
+    out = torch.empty(T, C, dtype=torch.bfloat16, device=u.device)
+    _lora_call("gnf4_hip_lora_up", u.device, u.data_ptr(), w.data_ptr(), transposed, w.shape[0],
+               C, r, *tb.args(), scale, base.data_ptr() if base is not None else None,
+               base.stride(0) if base is not None else 0, out.data_ptr(), out.stride(0))
+    return out
+
+
+def _lora_wgrad(p, q, like, transposed, tb, scale):
+    dw = torch.empty_like(like)
+    _lora_call("gnf4_hip_lora_wgrad", p.device, p.data_ptr(), p.stride(0), q.data_ptr(),
+               transposed, like.shape[0], p.shape[1], q.shape[1], tb.ids.data_ptr(),
+               tb.row_off.data_ptr(), tb.G, scale, dw.data_ptr())
+    return dw
+
+
+class _LoraAdd(torch.autograd.Function):
+    """``base + bf16(scaling * (a A[e]^T) B[e]^T)`` through the kernels of
+    csrc/gnf4_lora.hip (two forward, four backward launches, fp32 sums): the
+    values and gradients of adding ``lora_delta_grouped``. A backward that is
+    itself differentiated runs that torch composition instead."""
+
+    @staticmethod
+    def forward(ctx, base, a_cat, lora_A, lora_B, sizes, expert_ids, scaling):
+        a = nf4_grouped._act_view(a_cat.detach())
+        tb = _LoraTables(sizes, expert_ids, a.device)
+        u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
+        ctx.save_for_backward(a_cat, lora_A, lora_B, u)
+        ctx.tables, ctx.args = tb, (sizes, expert_ids, scaling)
+        return _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling),
+                        nf4_grouped._act_view(base))
+
+    @staticmethod
+    def backward(ctx, g):
+        a_cat, A, B, u = ctx.saved_tensors
+        sizes, expert_ids, scaling = ctx.args
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            with torch.enable_grad():
+                ins = [t for t, n in zip((a_cat, A, B), need[1:4]) if n]
+                d = lora_delta_grouped(a_cat, A, B, sizes, expert_ids, scaling).to(g.dtype)
+                got = iter(torch.autograd.grad(d, ins, g, create_graph=True) if ins else ())
+            return (g, *(next(got) if n else None for n in need[1:4]), None, None, None)
+        tb, s = ctx.tables, float(scaling)
+        gv = nf4_grouped._act_view(g)
+        gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
+        ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None
+        gA = _lora_wgrad(nf4_grouped._act_view(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
+        gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
+        return g, ga, gA, gB, None, None, None
+
+
 def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lora_B=None,
                        weights_fn=None, scaling=1.0, dgrad_kernel=True):
     """Frozen NF4 projection plus the trainable delta, pre-activation
@@ -206,5 +331,7 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
                                   weights_fn=weights_fn, dgrad_kernel=dgrad_kernel)
     if lora_A is None or lora_B is None:
         return out
+    if _kernels_take(out, a_cat, lora_A, lora_B, sizes):
+        return _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     delta = lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     return out if delta is None else out + delta.to(out.dtype)

@@ -52,7 +52,7 @@
 extern "C" {
 #endif
 
-#define GNF4_HIP_ABI_VERSION 14
+#define GNF4_HIP_ABI_VERSION 15
 
 #define GNF4_FMT_NF4 0
 #define GNF4_FMT_MXFP4 1
@@ -447,6 +447,36 @@ int gnf4_hip_gather_rows(const void *x, int64_t ldx, const int32_t *order, int64
 int gnf4_hip_route_combine(const void *y, int64_t ldy, const int32_t *pos,
                            const uint16_t *wts, int64_t wts_stride, int64_t T, int k,
                            int64_t D, void *out, int64_t ldo, void *stream);
+
+/* The low-rank half of a fine-tuned grouped projection, fp32 products over
+ * ragged groups (reference kernel/nf4_qlora.py:181-305, there torch batched
+ * matmuls over padded groups). Group g owns the rows row_off[g] ..
+ * row_off[g + 1] as tiles tile_off[g] .. tile_off[g + 1] of at most 16 rows;
+ * tile_off and row_off [G + 1], expert_ids [G], n_tiles = tile_off[G]; all
+ * int32 on the device; an id outside [0, E) contributes nothing. w [E, r, C]
+ * or [E, C, r] fp32 contiguous and 16-byte aligned, r <= 64 and r % 4 == 0;
+ * C, ldx, ldb, ldo, ldp % 8 == 0; x, base, out, p bf16, 16-byte aligned.
+ *
+ * y[t, j] = scale * sum_c x[t, c] w(c, j); y [T, r] fp32. transposed == 0: w
+ * is [E, r, C]; else [E, C, r]. */
+int gnf4_hip_lora_down(const void *x, int64_t ldx, const float *w, int transposed, int64_t E,
+                       int64_t C, int r, const int32_t *tile_off, const int32_t *row_off,
+                       const int32_t *expert_ids, int G, int n_tiles, float scale, float *y, void *stream);
+
+/* out[t, n] = bf16(scale * sum_j u[t, j] w(n, j)), added to base[t, n] (one
+ * more bf16 rounding) when base is not NULL; u [T, r] fp32. transposed == 0:
+ * w is [E, C, r]; else [E, r, C]. */
+int gnf4_hip_lora_up(const float *u, const float *w, int transposed, int64_t E, int64_t C, int r,
+                     const int32_t *tile_off, const int32_t *row_off, const int32_t *expert_ids,
+                     int G, int n_tiles, float scale, const void *base, int64_t ldb, void *out, int64_t ldo,
+                     void *stream);
+
+/* dw[e] = scale * sum over the rows t of e's groups of p[t, :] x q[t, :], for
+ * every e in [0, E) (zeros where no group has it); q [T, r] fp32. transposed == 0: dw is
+ * [E, C, r]; else [E, r, C]. */
+int gnf4_hip_lora_wgrad(const void *p, int64_t ldp, const float *q, int transposed, int64_t E,
+                        int64_t C, int r, const int32_t *expert_ids, const int32_t *row_off,
+                        int G, float scale, float *dw, void *stream);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,104 @@
+"""The low-rank kernels (csrc/gnf4_lora.hip) behind fused_grouped_lora: values
+and gradients against the torch composition of the same delta, and the calls
+that must keep taking that composition.
+
+Tolerances: the fp32 sums run in another order (contractions of at most 2048
+terms: relative error below 2048^0.5 * 2^-24 * a few, asserted at 1e-5); bf16
+outputs of sums that close differ only where a rounding flips, by one bf16 step
+(2^-8) in a small share of values: 1e-3 relative Frobenius error."""
+import pytest
+import torch
+
+from _fixtures import rand_nf4_stack, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(sizes, ids, E, K, N, r, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    T = sum(sizes)
+    W, S = rand_nf4_stack(E, N, K, seed)
+    x = rnd(T, K).to("cuda", torch.bfloat16)
+    A = (rnd(E, r, K) / K ** 0.5).cuda()
+    B = (rnd(E, N, r) * 0.3).cuda()
+    go = (rnd(T, N) * 0.1).to("cuda", torch.bfloat16)
+    return W, S, x, A, B, go
+
+
+def _run(kernels, W, S, x, A, B, go, sizes, ids, monkeypatch):
+    import nf4_qlora
+    if not kernels:
+        monkeypatch.setattr(nf4_qlora, "_kernels_take", lambda *a: False)
+    x, A, B = (t.detach().clone().requires_grad_(True) for t in (x, A, B))
+    out = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B, scaling=2.0)
+    grads = torch.autograd.grad(out, (x, A, B), go)
+    monkeypatch.undo()
+    return [out.detach(), *grads]
+
+
+@pytest.mark.parametrize("sizes,ids,E,K,N,r", [
+    ([5, 0, 17, 33, 1], [3, 1, 0, 2, 4], 6, 64, 64, 4),
+    ([16, 15, 31], [2, 0, 1], 3, 192, 72, 16),
+    ([40, 3, 20], [1, 1, 0], 3, 2048, 264, 12),          # one expert in two groups
+    ([64, 128], [0, 1], 2, 320, 520, 20),
+    ([70, 7], [1, 0], 2, 128, 1032, 64),
+    ([200] + [1] * 40, list(range(41)), 41, 64, 64, 8),  # far more padding than rows
+    ([2] * 130, list(range(130)), 131, 64, 64, 32),      # groups past two lane passes
+])
+@pytest.mark.parametrize("dev_ids", [False, True])
+def test_matches_the_torch_composition(sizes, ids, E, K, N, r, dev_ids, monkeypatch):
+    case = _case(sizes, ids, E, K, N, r)
+    arg = torch.tensor(ids, device="cuda") if dev_ids else ids
+    got = _run(True, *case, sizes, arg, monkeypatch)
+    want = _run(False, *case, sizes, ids, monkeypatch)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        assert rel_err(a, b.double()) <= (1e-3 if i < 2 else 1e-5), i
+    again = _run(True, *case, sizes, arg, monkeypatch)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+def test_route_and_the_calls_that_keep_the_torch_composition(monkeypatch):
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, go = _case(sizes, ids, 2, 128, 64, 8)
+    used = []
+    orig = nf4_qlora._LoraAdd.apply
+    monkeypatch.setattr(nf4_qlora._LoraAdd, "apply", lambda *a: used.append(1) or orig(*a))
+    run = lambda **k: nf4_qlora.fused_grouped_lora(  # noqa: E731
+        k.get("x", x), W, S, sizes, ids, k.get("A", A), k.get("B", B))
+    ref = run()
+    assert used == [1]
+    torch.testing.assert_close(run(A=A.double().float()), ref)
+    assert used == [1, 1]
+    # bf16 adapters, strided adapters, autocast, forward mode: the composition
+    run(A=A.bfloat16(), B=B.bfloat16())
+    strided = A.transpose(1, 2).contiguous().transpose(1, 2)
+    assert rel_err(run(A=strided), ref.double()) <= 1e-3
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        run()
+    with torch.autograd.forward_ad.dual_level():
+        d = run(A=torch.autograd.forward_ad.make_dual(A, torch.ones_like(A)))
+        assert torch.autograd.forward_ad.unpack_dual(d).tangent is not None
+    assert used == [1, 1]
+
+
+def test_double_backward_and_saved_tensor_hooks(monkeypatch):
+    """Gradients of gradients run through the torch composition; what is saved
+    goes through saved-tensor hooks."""
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, go = _case(sizes, ids, 2, 128, 64, 8)
+    res = []
+    for kernels in (True, False):
+        if not kernels:
+            monkeypatch.setattr(nf4_qlora, "_kernels_take", lambda *a: False)
+        a, b = A.clone().requires_grad_(True), B.clone().requires_grad_(True)
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t, lambda t: t):
+            out = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, a, b, scaling=2.0)
+        assert packed
+        ga, = torch.autograd.grad(out, a, go, create_graph=True)
+        res.append(torch.autograd.grad(ga.square().sum(), b)[0])
+    assert rel_err(res[0], res[1].double()) <= 1e-4
