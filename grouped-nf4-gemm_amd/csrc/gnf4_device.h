@@ -96,6 +96,16 @@ __device__ __forceinline__ void init_pair_table_imm(char* smem) {
   for (int j = 0; j < 16; ++j) tab[b * 32 + ((j0 + j + b) & 31)] = e;
 }
 
+// The same with 16 columns (32 KiB: entry (byte b, column c) at b * 128 + c * 8).
+__device__ __forceinline__ void init_pair_table16_imm(char* smem) {
+  const unsigned b = threadIdx.x & 255;
+  const float2 e = make_float2(nf4_code_imm(b >> 4), nf4_code_imm(b & 15));
+  const int j0 = threadIdx.x < 256 ? 0 : 8;
+  float2* tab = reinterpret_cast<float2*>(smem);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) tab[b * 16 + ((j0 + j + b) & 15)] = e;
+}
+
 __device__ __forceinline__ unsigned bf16x2_bits(float lo, float hi) {
   bf16x2_t r = {(__bf16)lo, (__bf16)hi};  // v_cvt_pk_bf16_f32, RNE
   return __builtin_bit_cast(unsigned, r);

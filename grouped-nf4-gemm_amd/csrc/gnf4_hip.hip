@@ -3732,8 +3732,8 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
   const int cus = device_cus();
   if (cus <= 0) return -2;
   {
-    // the four-wave tile with transposed tr8 reads of the packed rows: any
-    // tile of at most 256 rows, whole 64-wide n steps and 64-wide k blocks
+    // the tiles with transposed tr8 reads of the packed rows: at most 256
+    // rows, whole 64-wide n steps and 64-wide k blocks
     const bool w_ok = p.N % kDgStep == 0 && p.K % 64 == 0 && p.ldo % 4 == 0 &&
                       (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM &&
                       (int64_t)kPtBM * p.ldg * 2 < 0x7FFFFFFF &&
@@ -3754,15 +3754,31 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
       f.K = p.K;
       f.ldo = p.ldo;
       const int64_t tiles = (int64_t)p.n_mtiles * ((p.K + kPfBN - 1) / kPfBN);
+      const int64_t wide = (int64_t)p.n_mtiles * ((p.K + 2 * kPfBN - 1) / (2 * kPfBN));
       const int64_t per_x = prefill_w_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
+      // Two kernels with the same bits. A 512-column tile of k_tile_dgrad
+      // takes 1.3 (32 rows) to 1.75 (128 rows) times a 256-column tile of
+      // k_prefill_w, and two such 1.45 to 2 times as long, so it is taken
+      // where it needs at most 5/9 of the rounds of tiles over the CUs
+      // (128 experts, N = 2048, K = 768: 1 against 2 rounds, 75 against 89 us
+      // at 128 rows); with fewer tiles than that, CUs would stand idle.
+      const int64_t rounds = (tiles + cus - 1) / cus, wide_rounds = (wide + cus - 1) / cus;
+      if (block_m <= kPfBM && 9 * wide_rounds <= 5 * rounds) {
+        f.t_row0 = p.t_row0;
+        f.t_rows = p.t_rows;
+        f.t_group = p.t_group;
+        f.eids = p.eids;
+        return launch_tile_dgrad(FMT, f, p.out, tt ? *tt : no_tiles(),
+                                 prefill_w_per_xcd(wide, cus), stream);
+      }
       hipLaunchKernelGGL((k_prefill_w<FMT, true>), dim3((unsigned)(per_x * 8)), dim3(256), 0, stream,
                          f, p.t_row0, p.t_rows, p.t_group, p.eids, p.out, tt ? *tt : no_tiles());
       return hipGetLastError() == hipSuccess ? 0 : -2;
     }
   }
-  // a kernel-argument tile table is for the four-wave kernel only: the others
-  // read device tables
+  // a kernel-argument tile table is for those two only: the others read
+  // device tables
   if (tt) return -1;
   const bool tiled_ok = p.N % kDgStep == 0 && p.ldo % 4 == 0 &&
                         (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPfBM &&
@@ -4544,8 +4560,10 @@ int gnf4_hip_grouped_dgrad_tiles(int fmt, const void* grad_out, int g_dtype, int
   p.out = static_cast<uint16_t*>(out);
   p.ldo = ldo;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return fmt == GNF4_FMT_NF4 ? launch_dgrad<kNF4>(p, kPtBM, s, &tt)
-                             : launch_dgrad<kMX>(p, kPtBM, s, &tt);
+  int rows = 0;
+  for (int i = 0; i < n_mtiles; ++i) rows = tile_rows[i] > rows ? tile_rows[i] : rows;
+  return fmt == GNF4_FMT_NF4 ? launch_dgrad<kNF4>(p, rows, s, &tt)
+                             : launch_dgrad<kMX>(p, rows, s, &tt);
 }
 
 int gnf4_hip_nf4_dgrad(const void* grad_out, int g_dtype, int64_t ldg, const uint8_t* B,

@@ -1,5 +1,6 @@
-// gnf4_tile.hip -- the tiled forward of the grouped 4-bit expert GEMM on
-// gfx950: up to 256 token rows of one group x 256 weight rows per tile.
+// gnf4_tile.hip -- the eight-wave tile kernels of the grouped 4-bit expert
+// GEMM on gfx950: the forward (up to 256 token rows of one group x 256 weight
+// rows per tile) and the dgrad of groups of up to 128 rows (k_tile_dgrad).
 //
 // k_tile_fwd: eight waves (two per SIMD) on a persistent grid of one workgroup
 // per CU. Wave w owns 32 weight rows for all of the tile's token rows, so no
@@ -602,40 +603,53 @@ __device__ __forceinline__ int tile_fwd(const FwdArgs& p, const PfTile t, const 
   return run_a ? (slot0 + F) % kS : 0;
 }
 
+// A workgroup's share of the tile list: XCD x = blockIdx % 8 takes the x-th
+// contiguous eighth of it (m-tile major), its workgroups every stride-th tile
+// (tiles come largest first, so each gets one of every size band).
+struct TileWalk {
+  int width, n_tiles, idx, stride;
+  int64_t lo, hi;
+  __device__ __forceinline__ TileWalk(const FwdArgs& p, int cols, int col_tiles)
+      : width(cols), n_tiles(col_tiles) {
+    const int64_t total = (int64_t)p.n_mtiles * n_tiles;
+    const int nx = gridDim.x >= 8 ? 8 : 1;
+    const int x = (int)(blockIdx.x % nx);
+    idx = (int)(blockIdx.x / nx);
+    stride = (int)(gridDim.x / nx);
+    lo = total * x / nx;
+    hi = total * (x + 1) / nx;
+  }
+  // tile tg of the list; rows 0: none
+  __device__ __forceinline__ PfTile at(int64_t tg, const int32_t* __restrict__ t_row0,
+                                       const int32_t* __restrict__ t_rows,
+                                       const int32_t* __restrict__ t_group,
+                                       const int32_t* __restrict__ eids, const PwTiles& tt) const {
+    PfTile t{0, 0, 0, 0};
+    if (tg >= hi) return t;
+    const int mt = (int)(tg / n_tiles);
+    t.n0 = uniform((int)(tg - (int64_t)mt * n_tiles) * width);
+    if (tt.n > 0) {
+      t.row0 = uniform(tt.row0[mt]);
+      t.rows = uniform(tt.rows[mt]);
+      t.e = uniform(tt.grp_is_expert ? tt.grp[mt] : eids[tt.grp[mt]]);
+    } else {
+      t.row0 = uniform(t_row0[mt]);
+      t.rows = uniform(t_rows[mt]);
+      t.e = uniform(eids[t_group[mt]]);
+    }
+    return t;
+  }
+};
+
 template <int FMT>
 __global__ void __launch_bounds__(512, 2)
     k_tile_fwd(const FwdArgs p, const int32_t* __restrict__ t_row0,
                const int32_t* __restrict__ t_rows, const int32_t* __restrict__ t_group,
                const int32_t* __restrict__ eids, uint16_t* __restrict__ out, const PwTiles tt) {
   __shared__ __attribute__((aligned(16))) char smem[kTlLds];
-  const int n_tiles = (int)((p.N + kTlBN - 1) / kTlBN);
-  const int64_t total = (int64_t)p.n_mtiles * n_tiles;
-  const int nx = gridDim.x >= 8 ? 8 : 1;
-  const int x = (int)(blockIdx.x % nx), idx = (int)(blockIdx.x / nx);
-  const int stride = (int)(gridDim.x / nx);
-  const int64_t lo = total * x / nx, hi = total * (x + 1) / nx;
-  auto tile_at = [&](int64_t tg) {
-    PfTile t{0, 0, 0, 0};
-    if (tg >= hi) return t;   // rows 0: none
-    const int mt = (int)(tg / n_tiles);
-    t.n0 = (int)(tg - (int64_t)mt * n_tiles) * kTlBN;
-    if (tt.n > 0) {
-      t.row0 = tt.row0[mt];
-      t.rows = tt.rows[mt];
-      t.e = tt.grp_is_expert ? tt.grp[mt] : eids[tt.grp[mt]];
-    } else {
-      t.row0 = t_row0[mt];
-      t.rows = t_rows[mt];
-      t.e = eids[t_group[mt]];
-    }
-    t.row0 = uniform(t.row0);
-    t.rows = uniform(t.rows);
-    t.e = uniform(t.e);
-    t.n0 = uniform(t.n0);
-    return t;
-  };
-  int64_t tg = lo + idx;
-  PfTile t = tile_at(tg);
+  const TileWalk tw(p, kTlBN, (int)((p.N + kTlBN - 1) / kTlBN));
+  int64_t tg = tw.lo + tw.idx;
+  PfTile t = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
   if (t.rows <= 0) return;
   const int F = uniform((int)(p.K / kTlBK));
   TileRegs<FMT> regs;
@@ -649,8 +663,8 @@ __global__ void __launch_bounds__(512, 2)
   __builtin_amdgcn_s_barrier();
   int slot = 0;
   while (t.rows > 0) {
-    tg += stride;
-    const PfTile tn = tile_at(tg);
+    tg += tw.stride;
+    const PfTile tn = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
     switch ((t.rows + 31) >> 5) {
       case 8: slot = tile_fwd<FMT, 8>(p, t, tn, smem, out, regs, slot); break;
       case 7: slot = tile_fwd<FMT, 7>(p, t, tn, smem, out, regs, slot); break;
@@ -662,6 +676,399 @@ __global__ void __launch_bounds__(512, 2)
       default: slot = tile_fwd<FMT, 1>(p, t, tn, smem, out, regs, slot); break;
     }
     slot = uniform(slot);
+    t = tn;
+  }
+  // no load may write this workgroup's LDS after it ends
+  wait_vm_lgkm0<0>();
+}
+
+// ================================================================ dgrad ==
+//
+// k_tile_dgrad: out[t, k] = sum_n grad[t, n] W[e][n, k], tiles of up to 128
+// gradient rows of one group x 512 output columns (k), the contraction over n
+// in ascending steps of 64 packed rows. Eight waves, two per SIMD, of 64
+// columns each: no weight is decoded twice, and one wave's lookups run while
+// the other's MFMAs do. (One wave per SIMD, the 256-row kernel's form, waits
+// out every LDS round trip when a tile has few rows to hide it behind.)
+//   * gradient rows (two-deep) and packed rows and scales (three-deep) come
+//     through LDS rings by direct-to-LDS loads: one barrier per step both
+//     publishes the next step and frees the last;
+//   * one ds_read_b64_tr_b8 per 16-row slice hands each lane one byte column
+//     of 8 packed rows. Byte c holds k = 2 c (first nibble) and 2 c + 1, which
+//     feed the MFMA blocks 0 and 1: block b, MFMA row i is the wave's column
+//     2 i + b. The rows of the tr8 read come in the order 0,2,4,6,1,3,5,7, so
+//     dword 0 holds the even rows, dword 1 the odd ones, and the bf16 pair
+//     (row 2 m, row 2 m + 1) comes from byte m of each;
+//   * slice kk looks up the next slice's weights in its first half and packs
+//     them, each row by its own scale, in its second;
+//   * the loads run on into the workgroup's next tile.
+// The products of an output are added in the 256-row kernel's order: both
+// give the same bits.
+// What bounds it: at 128 rows the MFMAs (1024 clocks per wave and step, 2048
+// per SIMD) and the LDS (lookups, operand reads and stage writes, about 2400
+// clocks) half hide each other, a step takes 3800-4500; at 32 rows the chain
+// of lookup, pack and MFMA.
+// Measured (MI355X, 32 / 64 / 128 rows per group; before: the 256-row
+// kernel): NF4, 128 experts, N = 2048, K = 768: 45 / 54 / 75 us (67 / 69 / 89);
+// N = 1536, K = 2048: 71 / 88 / 119 (105 / 110 / 147); MXFP4, 32 experts,
+// N = 5760, K = 2880: 99 / 116 / 163 (177 / 177 / 201). Two halves of the step
+// list per tile instead of two tiles' columns: 49 / 59 / 80, and other bits.
+// A wave loading its own 32 bytes of every row: 133 us for MXFP4 at 32 rows.
+constexpr int kDtBM = 128;
+constexpr int kDtBN = 512;
+constexpr int kDtAct = kDtBM * kTlBK * 2;                   // a step's gradient rows
+constexpr int kDtRows = 64 * 128;                           // half a step's packed rows
+constexpr int kDtHalf = kDtRows + 2048;                     // and scales, a dword each
+constexpr int kDtWts = 2 * kDtHalf;                         // 20 KiB
+constexpr int kDtTab = 32 * 1024;                           // 16-column pair table
+constexpr int kDtW0 = kDtTab + 2 * kDtAct;                  // weight ring, three deep
+constexpr int kDtOut = kDtW0 + 3 * kDtWts;                  // per wave 32 rows x 64 columns
+static_assert(kDtOut + kTlWaves * 4096 <= kTlLds, "dgrad LDS");
+
+template <int FMT>
+struct DgradSrc {
+  const char* a;
+  const char* b;
+  const char* s;
+  int rows, a_bytes, b_bytes, s_bytes;
+  // columns [n0 + 256 half, +256), up to the last byte of the last row:
+  // columns past K read what follows their row (never stored), and zeros
+  // behind the expert's rows
+  __device__ __forceinline__ DgradSrc(const FwdArgs& p, const PfTile& t, int half) {
+    constexpr int kB = FMT == kNF4 ? 4 : 1, kBlk = FMT == kNF4 ? 64 : 32;
+    const int k0 = t.n0 + half * 256;
+    const bool live = t.rows > 0, in = live && k0 < p.K;
+    const int64_t k = in ? k0 : 0;
+    a = static_cast<const char*>(uniform_ptr(p.a + (int64_t)t.row0 * p.lda));
+    b = static_cast<const char*>(uniform_ptr(p.B + (int64_t)t.e * p.sbe + k / 2));
+    s = static_cast<const char*>(uniform_ptr(static_cast<const char*>(p.S) +
+                                             ((int64_t)t.e * p.sse + k / kBlk) * kB));
+    rows = t.rows;
+    a_bytes = uniform(live ? (int)((int64_t)t.rows * p.lda * 2) : 0);
+    b_bytes = uniform(in ? (int)((p.N - 1) * p.sbn + (p.K - k) / 2) : 0);
+    s_bytes = uniform(in ? (int)(((p.N - 1) * p.ssn + (p.K - k) / kBlk) * kB) : 0);
+  }
+};
+
+template <int FMT>
+struct DgradLoads {
+  static constexpr int kW = 2 + (FMT == kNF4 ? 1 : 2);   // weight loads per step
+  int a_voff[2], b_voff, s_voff, b_step, s_step, b_next, s_next;
+  __device__ __forceinline__ DgradLoads(const FwdArgs& p, int wave, int lane) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = (wave * 2 + i) * 8 + (lane >> 3);
+      a_voff[i] = (int)(row * p.lda * 2) + ((lane & 7) ^ pf_swz(row & 15)) * 16;
+    }
+    // the four waves of a half share its loads, so that neighbouring lanes
+    // read one row: 8 lanes its 128 packed bytes (16-byte chunk c of row r at
+    // c ^ (r % 8) in LDS), 4 lanes its absmax values, 8 its e8m0 bytes
+    const int w = wave & 3, l8 = lane >> 3;
+    b_voff = (int)((w * 16 + l8) * p.sbn) + ((lane & 7) ^ l8) * 16;
+    b_next = (int)(8 * p.sbn);
+    b_step = (int)(64 * p.sbn);
+    s_voff = FMT == kNF4 ? (int)((w * 16 + (lane >> 2)) * p.ssn + (lane & 3)) * 4
+                         : (int)((w * 16 + l8) * p.ssn) + (lane & 7);
+    s_next = (int)(8 * p.ssn);
+    s_step = (int)(64 * p.ssn * (FMT == kNF4 ? 4 : 1));
+  }
+  // gradient piece j (0, 1) of step g (of F); zeros for a step past the end,
+  // nothing for rows past the tile
+  __device__ __forceinline__ void act(char* smem, const DgradSrc<FMT>& x, int wave, int g, int F,
+                                      int slot, int j) const {
+    if ((wave * 2 + j) * 8 >= x.rows) return;
+    char* dst = smem + kDtTab + slot * kDtAct + (wave * 2 + j) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_of(x.a, g < F ? x.a_bytes : 0), (lds_ptr_t)dst,
+                                             16, a_voff[j], uniform(g * (kTlBK * 2)), 0, 0);
+  }
+  // weight load j (0..kW - 1) of step g: packed rows, then scales
+  __device__ __forceinline__ void wts(char* smem, const DgradSrc<FMT>& x, int wave, int g, int F,
+                                      int slot, int j) const {
+    char* w = smem + kDtW0 + slot * kDtWts + (wave >> 2) * kDtHalf;
+    const int q = wave & 3;
+    if (j < 2) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc_of(x.b, g < F ? x.b_bytes : 0), (lds_ptr_t)(w + (q * 2 + j) * 1024), 16, b_voff,
+          uniform(g < F ? g * b_step + j * b_next : 0), 0, 0);
+      return;
+    }
+    const __amdgpu_buffer_rsrc_t rs = rsrc_of(x.s, g < F ? x.s_bytes : 0);
+    if constexpr (FMT == kNF4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(w + kDtRows + q * 256), 4, s_voff,
+                                               uniform(g < F ? g * s_step : 0), 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(w + kDtRows + (q * 2 + j - 2) * 256), 1,
+                                               s_voff, uniform(g < F ? g * s_step + (j - 2) * s_next : 0), 0, 0);
+  }
+};
+
+// Ring positions: gradient slot 0..1, weight slot 0..2
+struct DgradPos {
+  int a, w;
+};
+
+// One tile. On entry its step 0 is at `at`, landed and published, and the
+// weights of its step 1 are on their way. Returns where tn's step 0 is, in
+// the same state.
+template <int FMT, int kM>
+__device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t, const PfTile tn,
+                                          char* smem, uint16_t* __restrict__ out, const DgradPos at) {
+  const int lane = opaque(threadIdx.x) & 63, wave = uniform(threadIdx.x >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  const int half = wave >> 2, w = wave & 3;
+  const int F = uniform((int)(p.N / kTlBK));
+  using L = DgradLoads<FMT>;
+  const DgradSrc<FMT> x(p, t, half), xn(p, tn, half);
+  const L ld(p, wave, lane);
+
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)smem;
+  const int a_off = kDtTab + l32 * 128 + ((4 * h) ^ pf_swz(l32 & 15)) * 16;
+  auto act_addr = [&](int slot, int kk) {
+    unsigned addr = lds0 + slot * kDtAct + (a_off ^ (kk * 16));
+    asm("" : "+v"(addr));
+    return addr;
+  };
+  // the tr8 read of slice kk: lane i of its 16-lane group supplies 8 bytes of
+  // row pi(i / 2), half i % 2 of the group's 16
+  const int w_off = kDtW0 + half * kDtHalf;
+  const int tr_row = ((lane >> 1) & 3) * 2 + ((lane >> 3) & 1);
+  const int tr_off = w_off + (32 * h + tr_row) * 128 +
+                     ((w * 2 + ((lane >> 4) & 1)) ^ tr_row) * 16 + (lane & 1) * 8;
+  // the scales of row 32 h (MXFP4: of the lane's 32-column block)
+  constexpr int kSRow = FMT == kNF4 ? 16 : 32;
+  const int s_off = w_off + kDtRows + 32 * h * kSRow +
+                    (FMT == kNF4 ? w : w * 2 + (l32 >> 4)) * 4;
+  // pair-table address << 1 | column * 16 (nf4_dword_to_bf16_t16's form)
+  const unsigned reg2 = (unsigned)(lane & 15) * 16u;
+
+  unsigned pw[2][4];      // packed dwords of a step's slices
+  auto read_w = [&](int slot) {
+    typedef __attribute__((address_space(3))) v2i32_t lds_v2i32;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const v2i32_t r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (lds_v2i32*)(lds_ptr_t)(smem + slot * kDtWts + tr_off + kk * 8 * 128));
+      pw[0][kk] = (unsigned)r.x;
+      pw[1][kk] = (unsigned)r.y;
+    }
+  };
+  u32x4_t wf[2][2];       // [slice parity][block]
+  f32x2_t tp[2][4];       // NF4: looked-up pairs of the target
+  unsigned tw[2];         // MXFP4: its dwords
+  unsigned ts[8];         // its rows' scales, as read
+  // half m2 (bytes 2 m2, 2 m2 + 1) of the target (slot, slice kk)
+  auto look = [&](int slot, int kk, int m2) {
+    if (m2 == 0) {
+      typedef __attribute__((address_space(3))) unsigned lds_u32;
+      lds_u32* sp = (lds_u32*)(lds_ptr_t)(smem + slot * kDtWts + s_off + kk * 8 * kSRow);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) ts[r] = sp[r * kSRow / 4];
+      if constexpr (FMT != kNF4) {
+        tw[0] = pw[0][kk];
+        tw[1] = pw[1][kk];
+      }
+    }
+    if constexpr (FMT == kNF4)
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int m = 2 * m2; m < 2 * m2 + 2; ++m)
+          tp[d][m] = lds_read8f(
+              __builtin_amdgcn_perm(pw[d][kk], reg2, 0x0C0C0000u | ((4u + m) << 8)) >> 1);
+  };
+  auto scale = [&](int r) -> float {
+    const unsigned v = ts[r];
+    if constexpr (FMT == kNF4) return __uint_as_float(v);
+    else return e8m0_to_f32(v & 0xFFu);
+  };
+  auto pack = [&](int par, int m2) {
+#pragma unroll
+    for (int m = 2 * m2; m < 2 * m2 + 2; ++m) {
+      const float s0 = scale(2 * m), s1 = scale(2 * m + 1);
+      if constexpr (FMT == kNF4) {
+        wf[par][0][m] = bf16x2_bits(tp[0][m].x * s0, tp[1][m].x * s1);
+        wf[par][1][m] = bf16x2_bits(tp[0][m].y * s0, tp[1][m].y * s1);
+      } else {
+        auto cvt = [&](unsigned v, float sc) {
+          bf16x2_t r;
+          if (m == 0) r = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc, 0);
+          else if (m == 1) r = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc, 1);
+          else if (m == 2) r = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc, 2);
+          else r = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v, sc, 3);
+          return __builtin_bit_cast(unsigned, r);
+        };
+        const unsigned c0 = cvt(tw[0], s0), c1 = cvt(tw[1], s1);
+        wf[par][0][m] = __builtin_amdgcn_perm(c1, c0, 0x05040100u);
+        wf[par][1][m] = __builtin_amdgcn_perm(c1, c0, 0x07060302u);
+      }
+    }
+  };
+
+  // ---- prologue: gradients of step 1, weights of step 2 (of the next tile's
+  // step 0 where this one has two), and slice 0 of step 0
+  int sa = at.a, sw = at.w;
+  auto next_w = [](int v) { return v == 2 ? 0 : v + 1; };
+  {
+    const int w2 = next_w(next_w(sw));
+    const bool cur = F != 2;
+    const DgradSrc<FMT>& y = cur ? x : xn;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ld.act(smem, x, wave, 1, F, sa ^ 1, j);
+#pragma unroll
+    for (int j = 0; j < L::kW; ++j) ld.wts(smem, y, wave, uniform(cur ? 2 : 0), F, w2, j);
+  }
+  read_w(sw);
+  look(sw, 0, 0);
+  look(sw, 0, 1);
+  pack(0, 0);
+  pack(0, 1);
+  u32x4_t av[kM];
+#pragma unroll
+  for (int i = 0; i < kM; ++i) av[i] = lds_read16(act_addr(sa, 0) + i * 4096);
+  f32x16_t acc[2][kM];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < kM; ++i) acc[b][i] = f32x16_t{};
+
+  for (int f = 0; f < F; ++f) {
+    const bool last = f + 1 >= F;
+    auto slice = [&](auto KI) {
+      constexpr int kk = decltype(KI)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kk == 3) {
+        // step f + 1 has landed (newer: the weights of step f + 2), and every
+        // wave has read all of step f's slots
+        wait_vm_lgkm0<L::kW>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        read_w(next_w(sw));
+      }
+      const int ts_slot = kk == 3 ? next_w(sw) : sw;
+      const unsigned src = act_addr(kk == 3 ? sa ^ 1 : sa, (kk + 1) & 3);
+      constexpr int n = 2 * kM;
+#pragma unroll
+      for (int i = 0; i < kM; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          acc[b][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              as_bf16x8(wf[kk & 1][b]), as_bf16x8(av[i]), acc[b][i], 0, 0, 0);
+          const int pos = 2 * i + b;
+          if (b == 1) av[i] = lds_read16(src + i * 4096);
+          // the gradients of step f + 2, then the weights of step f + 3 (past
+          // the end: the next tile's step 0, steps 0 and 1), into the slots
+          // that the barrier freed
+          if constexpr (kk == 3) {
+            if (!last) {
+              constexpr int kAll = 2 + L::kW;
+#pragma unroll
+              for (int j = 0; j < kAll; ++j) {
+                if ((j * n) / kAll != pos) continue;
+                const int g = f + (j < 2 ? 2 : 3);
+                const bool cur = g < F;
+                const DgradSrc<FMT>& y = cur ? x : xn;
+                if (j < 2) ld.act(smem, y, wave, uniform(cur ? g : g - F), F, sa, j);
+                else ld.wts(smem, y, wave, uniform(cur ? g : g - F), F, sw, j - 2);
+              }
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if ((q * n) / 4 != pos) continue;
+            if (q < 2) look(ts_slot, (kk + 1) & 3, q);
+            else pack((kk + 1) & 1, q - 2);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    slice(std::integral_constant<int, 0>{});
+    slice(std::integral_constant<int, 1>{});
+    slice(std::integral_constant<int, 2>{});
+    slice(std::integral_constant<int, 3>{});
+    sa ^= 1;
+    sw = next_w(sw);
+  }
+  // ---- epilogue. sa and sw (of step F) hold the next tile's step 0, landed
+  // and published, unless the tile had a single step. Each wave turns its own
+  // 32 x 64 subtiles through its own LDS, and stores whole 128-byte pieces.
+  __builtin_amdgcn_sched_barrier(0);
+  if (F == 1) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ld.act(smem, xn, wave, 0, F, sa, j);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int j = 0; j < L::kW; ++j) ld.wts(smem, xn, wave, g, F, g ? next_w(sw) : sw, j);
+  }
+  char* ob = smem + kDtOut + wave * 4096;
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+      uniform_ptr(out + (int64_t)t.row0 * p.ldo), 0, uniform((int)((int64_t)t.rows * p.ldo * 2)),
+      0x00020000);
+  const int ldo2 = (int)(p.ldo * 2);
+  const int col = t.n0 + wave * 64 + (lane & 7) * 8;
+  const int coff = col < p.K ? col * 2 + (lane >> 3) * ldo2 : kOOB;   // K % 64 == 0
+#pragma unroll
+  for (int i = 0; i < kM; ++i) {
+    // MFMA row 8 g + 4 h + q of block b is column 16 g + 8 h + 2 q + b
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u32x4_t v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = bf16x2_bits(acc[0][i][4 * g + q], acc[1][i][4 * g + q]);
+      *reinterpret_cast<u32x4_t*>(ob + l32 * 128 + (((2 * g + h) ^ (l32 & 7)) << 4)) = v;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = j * 8 + (lane >> 3);
+      const u32x4_t v =
+          *reinterpret_cast<const u32x4_t*>(ob + row * 128 + (((lane & 7) ^ (row & 7)) << 4));
+      store_b128(v, ro, coff, uniform((i * 32 + j * 8) * ldo2));
+    }
+  }
+  if (F == 1) {
+    wait_vm_lgkm0<0>();
+    __builtin_amdgcn_s_barrier();
+  }
+  return {sa, sw};
+}
+
+template <int FMT>
+__global__ void __launch_bounds__(512, 2)
+    k_tile_dgrad(const FwdArgs p, const int32_t* __restrict__ t_row0,
+                 const int32_t* __restrict__ t_rows, const int32_t* __restrict__ t_group,
+                 const int32_t* __restrict__ eids, uint16_t* __restrict__ out, const PwTiles tt) {
+  __shared__ __attribute__((aligned(16))) char smem[kTlLds];
+  const TileWalk tw(p, kDtBN, (int)((p.K + kDtBN - 1) / kDtBN));
+  int64_t tg = tw.lo + tw.idx;
+  PfTile t = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+  if (t.rows <= 0) return;
+  {
+    const int lane = opaque(threadIdx.x) & 63, wave = uniform(threadIdx.x >> 6);
+    const DgradSrc<FMT> x(p, t, wave >> 2);
+    const DgradLoads<FMT> ld(p, wave, lane);
+    const int F = uniform((int)(p.N / kTlBK));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ld.act(smem, x, wave, 0, F, 0, j);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int j = 0; j < DgradLoads<FMT>::kW; ++j) ld.wts(smem, x, wave, g, F, g, j);
+  }
+  if constexpr (FMT == kNF4) init_pair_table16_imm(smem);
+  wait_vm_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  DgradPos at{0, 0};
+  while (t.rows > 0) {
+    tg += tw.stride;
+    const PfTile tn = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+    switch ((t.rows + 31) >> 5) {
+      case 4: at = tile_dgrad<FMT, 4>(p, t, tn, smem, out, at); break;
+      case 3: at = tile_dgrad<FMT, 3>(p, t, tn, smem, out, at); break;
+      case 2: at = tile_dgrad<FMT, 2>(p, t, tn, smem, out, at); break;
+      default: at = tile_dgrad<FMT, 1>(p, t, tn, smem, out, at); break;
+    }
+    at.a = uniform(at.a);
+    at.w = uniform(at.w);
     t = tn;
   }
   // no load may write this workgroup's LDS after it ends
@@ -681,6 +1088,18 @@ int launch_tile_fwd(int fmt, const FwdArgs& p, const PwTiles& tt, int64_t per_x,
   else
     hipLaunchKernelGGL((k_tile_fwd<kMX>), grid, block, 0, stream, p, p.t_row0, p.t_rows,
                        p.t_group, p.eids, p.out, tt);
+  return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+int launch_tile_dgrad(int fmt, const FwdArgs& p, uint16_t* out, const PwTiles& tt, int64_t per_x,
+                      hipStream_t stream) {
+  const dim3 grid((unsigned)(per_x * 8)), block(64 * kTlWaves);
+  if (fmt == kNF4)
+    hipLaunchKernelGGL((k_tile_dgrad<kNF4>), grid, block, 0, stream, p, p.t_row0, p.t_rows,
+                       p.t_group, p.eids, out, tt);
+  else
+    hipLaunchKernelGGL((k_tile_dgrad<kMX>), grid, block, 0, stream, p, p.t_row0, p.t_rows,
+                       p.t_group, p.eids, out, tt);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -439,8 +439,7 @@ def _tiles_np(sizes_i, block_m: int):
 
 
 def _xcd_balanced(t_row0, t_rows, t_group):
-    """Order 256-row tiles for the four-wave kernels, which hand XCD x the
-    x-th contiguous eighth of the tile list: the tiles, largest height class
+    """Order tiles for the persistent kernels, which hand XCD x the x-th contiguous eighth of the tile list: the tiles, largest height class
     first (group order within a class), are dealt round robin to 8 bins,
     which then run back to back. Each bin gets an equal share of every
     class and runs its largest tiles first. Only the order changes; every
@@ -884,12 +883,18 @@ def _launch_fwd(fmt: int, a_cat, W, S, sizes, expert_ids, block_m, op, fp32w=Fal
     return out
 
 
+def _dgrad_transposed_ok(N: int, K: int) -> bool:
+    """Whole 64-wide n steps and k blocks: the persistent kernels that read
+    the packed rows transposed, which also take kernel-argument tables."""
+    return N % 64 == 0 and K % 64 == 0
+
+
 def _dgrad_block_m(max_rows: int, N: int, K: int) -> int:
-    """Tile height of a dgrad launch: 256-row tiles when the four-wave
-    transposed-read kernel takes the shape (whole 64-wide n steps and k
-    blocks), else the forward's group-size rule capped at 128 rows (the
-    eight-wave dgrad kernels)."""
-    if max_rows > 128 and N % 64 == 0 and K % 64 == 0:
+    """Tile height of a dgrad launch: 256 rows for groups above 128 where the
+    transposed-read kernels take the shape, else the forward's group-size
+    rule capped at 128 rows (which the 512-column tiles and the decoding
+    kernels need). The bits do not depend on it."""
+    if max_rows > 128 and _dgrad_transposed_ok(N, K):
         return 256
     return _kernel_block_m(_prefill_block_m(max_rows))
 
@@ -934,13 +939,14 @@ def _launch_dgrad(fmt: int, grad_out, W, S, sizes, expert_ids, op):
     # per-row arithmetic does not depend on it)
     bm = _dgrad_block_m(max(sizes_i), N, K)
     t0, tr, tg = _tiles_np(sizes_i, bm)
-    if bm == 256:
+    transposed = _dgrad_transposed_ok(N, K)
+    if transposed:
         t0, tr, tg = _xcd_balanced(t0, tr, tg)
     eids_dev = _eids_device(expert_ids, dev)
     if eids_dev is None:
         _check_host_ids(expert_ids, E)
     stream = _CurStream(dev)
-    if bm == 256 and len(t0) <= ARG_TILES_MAX:
+    if transposed and 0 < len(t0) <= ARG_TILES_MAX:
         a0, ar, ag, is_e, e_ptr = _arg_tiles(t0, tr, tg, eids_dev, expert_ids)
         with _device_ctx(dev):
             rc = lib.gnf4_hip_grouped_dgrad_tiles(

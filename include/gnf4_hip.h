@@ -34,10 +34,10 @@
  *   n_mtiles  > 0 -> tiled path: the tile table t_row0/t_rows/t_group
  *                    [n_mtiles] int32 (reference build_group_tiles,
  *                    kernel/nf4_grouped.py:334-362) with block_m in
- *                    {16, 32, 64, 128, 256}; t_rows[i] <= block_m. 256
- *                    selects the four-wave tall-tile kernel and needs
+ *                    {16, 32, 64, 128, 256}; t_rows[i] <= block_m. With
  *                    K % 64 == 0, N % 4 == 0, ldo % 4 == 0 and an 8-byte
- *                    aligned out (-1 otherwise). The tile order is free
+ *                    aligned out every height runs the eight-wave tile
+ *                    kernel; 256 needs them (-1 otherwise). The order is free
  *                    (each XCD takes a contiguous eighth of the list).
  *
  * Return codes (the reference CPU tier's convention, gnf4_native/cpu_kernels.c:745-761):
@@ -343,9 +343,10 @@ int gnf4_hip_nf4_ffn_noalloc_reset(uint32_t *error_word, void *stream);
  * contracting over N in fixed 64-wide ascending steps (output bits do not
  * depend on block_m). grad_out is [T, ldg] bf16, out is [T, ldo] bf16 with
  * ldo >= K. Tile table as for the forward tiled path (n_mtiles may be 0:
- * nothing to do). With N % 64 == 0 and K % 64 == 0 any block_m up to 256
- * runs the four-wave transposed-read kernel; other shapes need
- * block_m <= 128 (-1 otherwise). */
+ * nothing to do). With N % 64 == 0 and K % 64 == 0 any block_m up to 256 is
+ * taken by the persistent kernels that read the packed rows transposed (512
+ * columns per tile for block_m <= 128 where enough tiles fill the device);
+ * other shapes need block_m <= 128 (-1 otherwise). */
 int gnf4_hip_grouped_dgrad(int fmt, const void *grad_out, int g_dtype, int64_t ldg,
                            const uint8_t *B, int64_t stride_be, int64_t stride_bn,
                            const void *scales, int64_t stride_se, int64_t stride_sn,
@@ -354,7 +355,7 @@ int gnf4_hip_grouped_dgrad(int fmt, const void *grad_out, int g_dtype, int64_t l
                            int block_m, int64_t N, int64_t K, void *out, int64_t ldo,
                            void *stream);
 
-/* Grouped dgrad on 256-row tiles with the tile table in host memory, in the
+/* Grouped dgrad on tiles of up to 256 rows with the table in host memory, in the
  * kernel's arguments (as gnf4_hip_grouped_fwd_tiles): same bits as
  * gnf4_hip_grouped_dgrad with the same table. Needs N % 64 == 0 and
  * K % 64 == 0 (-1 otherwise); returns 1 without launching when

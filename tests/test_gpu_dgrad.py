@@ -191,3 +191,56 @@ def test_dgrad_tall_several_tiles_per_workgroup(fmt):
         dec = dequant(fmt, W[ids[g]], S[ids[g]]).to(torch.bfloat16)
         rows = torch.arange(T, device="cuda")
         assert torch.equal(got[g * T:(g + 1) * T], dec[rows % N]), g
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
+@pytest.mark.parametrize("G,N,K,rows,pads", [
+    (150, 64, 320, (1, 31, 32, 33), (0, 0, 0, 0)),        # one step, half a 512-column tile
+    (150, 128, 576, (64, 65, 96, 128), (8, 4, 1, 4)),     # two steps, a 64-column tail tile
+    (150, 192, 512, (127, 97, 2, 128), (16, 20, 3, 8)),
+    (300, 320, 1024, (128, 5, 63, 34), (0, 16, 2, 64)),   # several tiles per workgroup
+])
+def test_dgrad_wide_tiles_give_the_tall_kernels_bits(fmt, G, N, K, rows, pads):
+    """Tables of at most 128 rows over enough groups run 512-column tiles;
+    256-row tables the 256-row kernel. Both add an output's products in the
+    same order, so the bits agree, with padded rows in every operand and
+    groups on both sides of each 32-row subtile. Against fp64: one bf16
+    rounding of the weights and one of the result (2^-8 each, relative to the
+    sum of magnitudes) and N fp32 additions."""
+    import _hiplib
+    W, S = _stack(fmt, 8, N, K, seed=21)
+    sizes = [rows[g % 4] for g in range(G)]
+    T = sum(sizes)
+    pg, pb, ps, po = pads
+
+    def padded(x, pad):
+        buf = torch.full((*x.shape[:-1], x.shape[-1] + pad), 7, dtype=x.dtype, device="cuda")
+        buf[..., :x.shape[-1]] = x
+        return buf[..., :x.shape[-1]]
+
+    go, Wp, Sp = padded(rand_acts(T, N, seed=22), pg), padded(W, pb), padded(S, ps)
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    ids = [(3 * g) % 8 for g in range(G)]
+    row0 = [0]
+    for m in sizes[:-1]:
+        row0.append(row0[-1] + m)
+    eids, t0, tr, tg = dev(ids), dev(row0), dev(sizes), dev(list(range(G)))
+    lib = _hiplib.load()
+    outs = []
+    for bm in (128, 256):
+        out = torch.full((T, K + po), 7.0, dtype=torch.bfloat16, device="cuda")
+        rc = lib.gnf4_hip_grouped_dgrad(
+            0 if fmt == "nf4" else 1, go.data_ptr(), _hiplib.DTYPE_BF16, go.stride(0),
+            Wp.data_ptr(), Wp.stride(0), Wp.stride(1), Sp.data_ptr(), Sp.stride(0), Sp.stride(1),
+            eids.data_ptr(), t0.data_ptr(), tr.data_ptr(), tg.data_ptr(), G, bm, N, K,
+            out.data_ptr(), out.stride(0), torch.cuda.current_stream().cuda_stream)
+        _hiplib.check(rc, "dgrad")
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    assert bool((outs[0][:, K:] == 7).all())
+    n = sum(sizes[:8])
+    w = [dequant(fmt, W[e], S[e]).double() for e in ids[:8]]
+    a = go[:n].double().split(sizes[:8])
+    ref = torch.cat([x @ y for x, y in zip(a, w)])
+    mag = torch.cat([x.abs() @ y.abs() for x, y in zip(a, w)])
+    assert bool(((outs[0][:n, :K].double() - ref).abs() <= (2 * 2 ** -8 + N * 2 ** -24) * mag).all())
