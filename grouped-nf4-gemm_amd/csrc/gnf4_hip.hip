@@ -3764,7 +3764,7 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
       // (128 experts, N = 2048, K = 768: 1 against 2 rounds, 75 against 89 us
       // at 128 rows); with fewer tiles than that, CUs would stand idle.
       const int64_t rounds = (tiles + cus - 1) / cus, wide_rounds = (wide + cus - 1) / cus;
-      if (block_m <= kPfBM && 9 * wide_rounds <= 5 * rounds) {
+      if (block_m <= kDgradWideRows && 9 * wide_rounds <= 5 * rounds) {
         f.t_row0 = p.t_row0;
         f.t_rows = p.t_rows;
         f.t_group = p.t_group;

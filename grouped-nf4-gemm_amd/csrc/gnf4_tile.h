@@ -10,8 +10,9 @@ namespace gnf4 {
 int launch_tile_fwd(int fmt, const FwdArgs& p, const PwTiles& tt, int64_t per_x,
                     hipStream_t stream);
 
-// Dgrad tiles of at most 128 rows x 512 columns (p.a the gradient rows,
+// Dgrad tiles of at most kDgradWideRows rows x 512 columns (p.a the gradient rows,
 // N % 64 == 0 and K % 64 == 0), the same grid.
+constexpr int kDgradWideRows = 160;
 int launch_tile_dgrad(int fmt, const FwdArgs& p, uint16_t* out, const PwTiles& tt, int64_t per_x,
                       hipStream_t stream);
 

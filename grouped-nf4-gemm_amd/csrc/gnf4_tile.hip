@@ -714,7 +714,7 @@ __global__ void __launch_bounds__(512, 2)
 // N = 5760, K = 2880: 99 / 116 / 163 (177 / 177 / 201). Two halves of the step
 // list per tile instead of two tiles' columns: 49 / 59 / 80, and other bits.
 // A wave loading its own 32 bytes of every row: 133 us for MXFP4 at 32 rows.
-constexpr int kDtBM = 128;
+constexpr int kDtBM = kDgradWideRows;
 constexpr int kDtBN = 512;
 constexpr int kDtAct = kDtBM * kTlBK * 2;                   // a step's gradient rows
 constexpr int kDtRows = 64 * 128;                           // half a step's packed rows
@@ -722,8 +722,9 @@ constexpr int kDtHalf = kDtRows + 2048;                     // and scales, a dwo
 constexpr int kDtWts = 2 * kDtHalf;                         // 20 KiB
 constexpr int kDtTab = 32 * 1024;                           // 16-column pair table
 constexpr int kDtW0 = kDtTab + 2 * kDtAct;                  // weight ring, three deep
-constexpr int kDtOut = kDtW0 + 3 * kDtWts;                  // per wave 32 rows x 64 columns
-static_assert(kDtOut + kTlWaves * 4096 <= kTlLds, "dgrad LDS");
+constexpr int kDtActLoads = (kDtAct / 1024 + kTlWaves - 1) / kTlWaves;
+constexpr int kDtOut = kDtW0 + 3 * kDtWts;                  // per wave 16 rows x 64 columns
+static_assert(kDtOut + kTlWaves * 2048 <= kTlLds, "dgrad LDS");
 
 template <int FMT>
 struct DgradSrc {
@@ -753,13 +754,12 @@ struct DgradSrc {
 template <int FMT>
 struct DgradLoads {
   static constexpr int kW = 2 + (FMT == kNF4 ? 1 : 2);   // weight loads per step
-  int a_voff[2], b_voff, s_voff, b_step, s_step, b_next, s_next;
+  int a_voff, a_piece, b_voff, s_voff, b_step, s_step, b_next, s_next;
   __device__ __forceinline__ DgradLoads(const FwdArgs& p, int wave, int lane) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = (wave * 2 + i) * 8 + (lane >> 3);
-      a_voff[i] = (int)(row * p.lda * 2) + ((lane & 7) ^ pf_swz(row & 15)) * 16;
-    }
+    // piece j of a wave: rows (8 j + wave) 8 + lane / 8
+    const int row = wave * 8 + (lane >> 3);
+    a_voff = (int)(row * p.lda * 2) + ((lane & 7) ^ pf_swz(row & 15)) * 16;
+    a_piece = (int)(kTlWaves * 8 * p.lda * 2);
     // the four waves of a half share its loads, so that neighbouring lanes
     // read one row: 8 lanes its 128 packed bytes (16-byte chunk c of row r at
     // c ^ (r % 8) in LDS), 4 lanes its absmax values, 8 its e8m0 bytes
@@ -772,14 +772,14 @@ struct DgradLoads {
     s_next = (int)(8 * p.ssn);
     s_step = (int)(64 * p.ssn * (FMT == kNF4 ? 4 : 1));
   }
-  // gradient piece j (0, 1) of step g (of F); zeros for a step past the end,
+  // gradient piece j (of kDtActLoads) of step g (of F); zeros for a step past the end,
   // nothing for rows past the tile
   __device__ __forceinline__ void act(char* smem, const DgradSrc<FMT>& x, int wave, int g, int F,
                                       int slot, int j) const {
-    if ((wave * 2 + j) * 8 >= x.rows) return;
-    char* dst = smem + kDtTab + slot * kDtAct + (wave * 2 + j) * 1024;
+    if ((j * kTlWaves + wave) * 8 >= x.rows) return;
+    char* dst = smem + kDtTab + slot * kDtAct + (j * kTlWaves + wave) * 1024;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_of(x.a, g < F ? x.a_bytes : 0), (lds_ptr_t)dst,
-                                             16, a_voff[j], uniform(g * (kTlBK * 2)), 0, 0);
+                                             16, a_voff, uniform(j * a_piece + g * (kTlBK * 2)), 0, 0);
   }
   // weight load j (0..kW - 1) of step g: packed rows, then scales
   __device__ __forceinline__ void wts(char* smem, const DgradSrc<FMT>& x, int wave, int g, int F,
@@ -913,7 +913,7 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
     const bool cur = F != 2;
     const DgradSrc<FMT>& y = cur ? x : xn;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) ld.act(smem, x, wave, 1, F, sa ^ 1, j);
+    for (int j = 0; j < kDtActLoads; ++j) ld.act(smem, x, wave, 1, F, sa ^ 1, j);
 #pragma unroll
     for (int j = 0; j < L::kW; ++j) ld.wts(smem, y, wave, uniform(cur ? 2 : 0), F, w2, j);
   }
@@ -960,15 +960,15 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
           // that the barrier freed
           if constexpr (kk == 3) {
             if (!last) {
-              constexpr int kAll = 2 + L::kW;
+              constexpr int kAct = kDtActLoads, kAll = kAct + L::kW;
 #pragma unroll
               for (int j = 0; j < kAll; ++j) {
                 if ((j * n) / kAll != pos) continue;
-                const int g = f + (j < 2 ? 2 : 3);
+                const int g = f + (j < kAct ? 2 : 3);
                 const bool cur = g < F;
                 const DgradSrc<FMT>& y = cur ? x : xn;
-                if (j < 2) ld.act(smem, y, wave, uniform(cur ? g : g - F), F, sa, j);
-                else ld.wts(smem, y, wave, uniform(cur ? g : g - F), F, sw, j - 2);
+                if (j < kAct) ld.act(smem, y, wave, uniform(cur ? g : g - F), F, sa, j);
+                else ld.wts(smem, y, wave, uniform(cur ? g : g - F), F, sw, j - kAct);
               }
             }
           }
@@ -994,13 +994,13 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
   __builtin_amdgcn_sched_barrier(0);
   if (F == 1) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) ld.act(smem, xn, wave, 0, F, sa, j);
+    for (int j = 0; j < kDtActLoads; ++j) ld.act(smem, xn, wave, 0, F, sa, j);
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int j = 0; j < L::kW; ++j) ld.wts(smem, xn, wave, g, F, g ? next_w(sw) : sw, j);
   }
-  char* ob = smem + kDtOut + wave * 4096;
+  char* ob = smem + kDtOut + wave * 2048;
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(out + (int64_t)t.row0 * p.ldo), 0, uniform((int)((int64_t)t.rows * p.ldo * 2)),
       0x00020000);
@@ -1010,19 +1010,25 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
 #pragma unroll
   for (int i = 0; i < kM; ++i) {
     // MFMA row 8 g + 4 h + q of block b is column 16 g + 8 h + 2 q + b
+    u32x4_t v[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      u32x4_t v;
+    for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = bf16x2_bits(acc[0][i][4 * g + q], acc[1][i][4 * g + q]);
-      *reinterpret_cast<u32x4_t*>(ob + l32 * 128 + (((2 * g + h) ^ (l32 & 7)) << 4)) = v;
-    }
+      for (int q = 0; q < 4; ++q) v[g][q] = bf16x2_bits(acc[0][i][4 * g + q], acc[1][i][4 * g + q]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int row = j * 8 + (lane >> 3);
-      const u32x4_t v =
-          *reinterpret_cast<const u32x4_t*>(ob + row * 128 + (((lane & 7) ^ (row & 7)) << 4));
-      store_b128(v, ro, coff, uniform((i * 32 + j * 8) * ldo2));
+    for (int r16 = 0; r16 < 2; ++r16) {
+      if ((l32 >> 4) == r16)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<u32x4_t*>(ob + (l32 & 15) * 128 + (((2 * g + h) ^ (l32 & 7)) << 4)) =
+              v[g];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int row = j * 8 + (lane >> 3);
+        const u32x4_t o =
+            *reinterpret_cast<const u32x4_t*>(ob + row * 128 + (((lane & 7) ^ (row & 7)) << 4));
+        store_b128(o, ro, coff, uniform((i * 32 + r16 * 16 + j * 8) * ldo2));
+      }
     }
   }
   if (F == 1) {
@@ -1048,7 +1054,7 @@ __global__ void __launch_bounds__(512, 2)
     const DgradLoads<FMT> ld(p, wave, lane);
     const int F = uniform((int)(p.N / kTlBK));
 #pragma unroll
-    for (int j = 0; j < 2; ++j) ld.act(smem, x, wave, 0, F, 0, j);
+    for (int j = 0; j < kDtActLoads; ++j) ld.act(smem, x, wave, 0, F, 0, j);
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
@@ -1062,6 +1068,7 @@ __global__ void __launch_bounds__(512, 2)
     tg += tw.stride;
     const PfTile tn = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
     switch ((t.rows + 31) >> 5) {
+      case 5: at = tile_dgrad<FMT, 5>(p, t, tn, smem, out, at); break;
       case 4: at = tile_dgrad<FMT, 4>(p, t, tn, smem, out, at); break;
       case 3: at = tile_dgrad<FMT, 3>(p, t, tn, smem, out, at); break;
       case 2: at = tile_dgrad<FMT, 2>(p, t, tn, smem, out, at); break;

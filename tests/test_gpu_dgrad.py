@@ -244,3 +244,28 @@ def test_dgrad_wide_tiles_give_the_tall_kernels_bits(fmt, G, N, K, rows, pads):
     ref = torch.cat([x @ y for x, y in zip(a, w)])
     mag = torch.cat([x.abs() @ y.abs() for x, y in zip(a, w)])
     assert bool(((outs[0][:n, :K].double() - ref).abs() <= (2 * 2 ** -8 + N * 2 ** -24) * mag).all())
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
+@pytest.mark.parametrize("rows", [(129, 160, 1, 145), (130, 161, 96, 33)])
+@pytest.mark.parametrize("N", [64, 128, 320])
+def test_dgrad_wide_tiles_up_to_160_rows(fmt, rows, N, monkeypatch):
+    """A table in the kernel's arguments shows its largest tile: up to 160 rows
+    run 512-column tiles (161 do not). The uploaded 256-row table runs the
+    256-row kernel: the same bits, and fp64 within one bf16 rounding of the
+    weights, one of the result and N fp32 additions."""
+    import nf4_grouped
+    G, K = 150, 576
+    W, S = _stack(fmt, 8, N, K, seed=31)
+    sizes = [rows[g % 4] for g in range(G)]
+    ids = [(5 * g) % 8 for g in range(G)]
+    go = rand_acts(sum(sizes), N, seed=32)
+    got = _ops()[fmt](go, W, S, sizes, ids)
+    monkeypatch.setattr(nf4_grouped, "ARG_TILES_MAX", 0)
+    assert torch.equal(got, _ops()[fmt](go, W, S, sizes, ids))
+    n = sum(sizes[:4])
+    w = [dequant(fmt, W[e], S[e]).double() for e in ids[:4]]
+    a = go[:n].double().split(sizes[:4])
+    ref = torch.cat([x @ y for x, y in zip(a, w)])
+    mag = torch.cat([x.abs() @ y.abs() for x, y in zip(a, w)])
+    assert bool(((got[:n].double() - ref).abs() <= (2 * 2 ** -8 + N * 2 ** -24) * mag).all())
