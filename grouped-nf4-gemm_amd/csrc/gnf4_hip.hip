@@ -1961,9 +1961,7 @@ constexpr int kPfBN = 256;
 constexpr int kPfBK = 64;
 constexpr int kPfStage = kPfBM * kPfBK * 2; // bytes per LDS stage
 
-
-
-// 256-row tiles (k_prefill_w below).
+// 256-row tiles (k_dgrad_tall below).
 constexpr int kPtBM = 256;
 constexpr int kPtStage = kPtBM * kPfBK * 2;
 
@@ -1992,48 +1990,36 @@ __device__ __forceinline__ u32x4_t nf4_dword_to_bf16_t16(const char* lds0, unsig
   return r;
 }
 
-// ==================================================== four-wave prefill ==
+// ====================================================== four-wave dgrad ==
 //
-// k_prefill_w<FMT>: the tall-tile forward (256 token rows of one group x 256
-// weight rows per tile), 256-thread workgroups, one workgroup per CU and one
-// wave per SIMD. Each wave owns 64 weight rows (two 32-row MFMA
-// blocks) for all 256 token rows, so
-//   * every activation operand read from LDS feeds two MFMAs (half the LDS
-//     operand traffic of a 32-row-per-wave split), and
+// k_dgrad_tall<FMT>: dgrad tiles of 256 gradient rows of one group x 256 output
+// columns (k), 256-thread workgroups, one workgroup per CU and one wave per
+// SIMD. Each wave owns 64 columns (two 32-column MFMA blocks) for all of the
+// tile's rows, so
+//   * every gradient operand read from LDS feeds two MFMAs, and
 //   * a wave has the whole register file: 256 accumulator registers and room
 //     to decode the next step's weights while this step's MFMAs run.
 // Everything a step touches comes through LDS rings filled by direct-to-LDS
-// loads two steps ahead (activation stages, and per wave the packed weight
+// loads two steps ahead (gradient stages, and per wave the packed weight
 // bytes and scales), so the step loop is not unrolled over ring slots and
 // the accumulators keep fixed registers.
-// The decode of a k-slice is interleaved with the MFMAs of the following
-// slice ("rolling" decode): during slice 0 of step f the wave decodes slice 3
-// of step f, during slices 1..3 it decodes slices 0..2 of step f + 1, each
-// into the operand registers the previous slice's MFMAs released.
-// The grid is persistent (by default one workgroup per CU): each XCD
-// (workgroup ids go to the XCDs round robin) works through a contiguous
-// range of the m-tile-major tile list, its workgroups taking every
-// (workgroups per XCD)-th tile of it; the NF4 pair table is built once per
-// workgroup.
-// The k order of every output element is that of k_prefill, so both give
-// identical bits. A tile runs MFMAs and operand reads for its own 32-row
-// subtiles only (one instantiation per count, 2..8).
+// The decode of a slice is interleaved with the MFMAs of the following slice
+// ("rolling" decode): during slice 0 of step f the wave decodes slice 3 of
+// step f, during slices 1..3 it decodes slices 0..2 of step f + 1, each into
+// the operand registers the previous slice's MFMAs released.
+// The grid is persistent (one workgroup per CU): each XCD (workgroup ids go
+// to the XCDs round robin) works through a contiguous range of the
+// m-tile-major tile list, its workgroups taking every (workgroups per XCD)-th
+// tile of it; the NF4 pair table is built once per workgroup. A tile runs
+// MFMAs and operand reads for its own 32-row subtiles only (one instantiation
+// per count, 2..8).
+// Groups of up to 160 rows run k_tile_dgrad instead where its wider tiles
+// need few enough rounds; at 256 rows per group this kernel is the faster
+// (128 experts, N = 2048, K = 768: 119 us against 150 for the eight-wave form
+// in two 128-row parts).
 //
-// LDS map: activation stages at 0, 32 and 64 KiB; weight ring at 96 KiB
-// (three 10 KiB slots: 8 KiB of packed bytes, then the scales); the 16-column
-// NF4 pair table at 128 KiB.
-constexpr int kPwWaves = 4;
-constexpr int kPwRowsPerWave = kPtBM / kPwWaves;           // 64 activation rows staged per wave
-constexpr int kPwAPieces = kPtStage / 1024 / kPwWaves;     // 8 direct-to-LDS loads per wave
-constexpr int kPwW0 = 3 * kPtStage;                        // weight ring
-constexpr int kPwWSlot = 10 * 1024;                     // 8 KiB packed bytes + 4 waves x 2 x 256 B scales
-constexpr int kPwTab = 0x20000;                            // 16-column pair table
-constexpr int kPwLds = kPwTab + 256 * 16 * 8;              // 160 KiB
-static_assert(kPwW0 + 3 * kPwWSlot <= kPwTab, "weight ring below the pair table");
-
-// DG = true: the dgrad form, out[t, k] = sum_n grad[t, n] W[e][n, k]. The
-// grad rows stage like the forward's activations (the contraction runs over
-// n), t.n0 is the first output column k, and wave w owns the 64 columns
+// out[t, k] = sum_n grad[t, n] W[e][n, k]: the contraction runs over n, t.n0
+// is the first output column k, and wave w owns the 64 columns
 // [t.n0 + 64 w, +64). Its weight operands come from the packed rows read
 // transposed: per step the wave's slot holds 64 rows (n) x 32 bytes (its 64
 // k), and one ds_read_b64_tr_b8 per slice hands each lane one byte column c
@@ -2047,25 +2033,35 @@ static_assert(kPwW0 + 3 * kPwWSlot <= kPwTab, "weight ring below the pair table"
 // absmax of (row, the wave's 64-block) is staged per step as 64 floats.
 // MXFP4 (low nibble = even k) converts each row's byte with that row's e8m0
 // scale of the lane's 32-column block and pairs rows with a byte permute.
-template <int FMT, int kM, bool DG>
-__device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t, char* smem,
+//
+// LDS map: gradient stages at 0, 32 and 64 KiB; weight ring at 96 KiB
+// (three 10 KiB slots: 8 KiB of packed bytes, then the scales); the 16-column
+// NF4 pair table at 128 KiB.
+constexpr int kPwWaves = 4;
+constexpr int kPwRowsPerWave = kPtBM / kPwWaves;           // 64 activation rows staged per wave
+constexpr int kPwAPieces = kPtStage / 1024 / kPwWaves;     // 8 direct-to-LDS loads per wave
+constexpr int kPwW0 = 3 * kPtStage;                        // weight ring
+constexpr int kPwWSlot = 10 * 1024;                     // 8 KiB packed bytes + 4 waves x 2 x 256 B scales
+constexpr int kPwTab = 0x20000;                            // 16-column pair table
+constexpr int kPwLds = kPwTab + 256 * 16 * 8;              // 160 KiB
+static_assert(kPwW0 + 3 * kPwWSlot <= kPwTab, "weight ring below the pair table");
+
+template <int FMT, int kM>
+__device__ __forceinline__ void dgrad_tall_tile(const FwdArgs& p, const PfTile t, char* smem,
                                                uint16_t* __restrict__ out, const int lut,
                                                const bool build_table) {
   const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
   const int l32 = lane & 31, h = lane >> 5;
   constexpr int kScaleBytes = FMT == kNF4 ? 4 : 1;
-  // contraction length (forward: K; dgrad: N) and output width (N; K)
-  const int64_t Kc = DG ? p.N : p.K;
-  const int64_t Nout = DG ? p.K : p.N;
-  const int F = (int)((Kc + kPfBK - 1) / kPfBK);
+  const int F = (int)(p.N / kPfBK);   // steps of the contraction
   // per step: activation pieces, 2 weight-byte loads, scale loads (NF4: one
   // of 64 rows; MXFP4: two of 32 rows x 2 blocks)
   constexpr int kGroupLoads = kPwAPieces + 2 + (FMT == kNF4 ? 1 : 2);
   // table address << 1 | column * 16 (nf4_dword_to_bf16_t16)
   const unsigned reg2 = ((unsigned)kPwTab << 1) | (unsigned)(lane & 15) * 16u;
 
-  // k mapping within a 64-wide step (as in k_prefill): lane half h covers
-  // k [32 h, 32 h + 32); MFMA slice kk takes k [32 h + 8 kk, +8).
+  // n mapping within a 64-wide step: lane half h covers
+  // n [32 h, 32 h + 32); MFMA slice kk takes n [32 h + 8 kk, +8).
   int a_off[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) a_off[kk] = l32 * 128 + ((4 * h + kk) ^ pf_swz(l32 & 15)) * 16;
@@ -2087,37 +2083,20 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   const int b_bytes = (int)(p.N * p.sbn);
   const int s_bytes = (int)(p.N * p.ssn * kScaleBytes);
   int b_voff[2], s_voff[2];
-  if constexpr (DG) {
-    // step rows n0 + 32 rb + lane / 2, 16 bytes (lane % 2) of the wave's 32;
-    // per step only soffset (n0 rows) moves. A wave past K loads zeros.
-    const int64_t kw = t.n0 + wave * 64;
+  // step rows n0 + 32 rb + lane / 2, 16 bytes (lane % 2) of the wave's 32;
+  // per step only soffset (n0 rows) moves. A wave past K loads zeros.
+  const int64_t kw = t.n0 + wave * 64;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-      b_voff[rb] = kw < p.K ? (int)((rb * 32 + (lane >> 1)) * p.sbn + kw / 2) + (lane & 1) * 16 : kOOB;
-    if constexpr (FMT == kNF4) {
-      s_voff[0] = kw < p.K ? (int)(lane * p.ssn * 4 + (kw >> 6) * 4) : kOOB;
-      s_voff[1] = kOOB;
-    } else {
-      // two e8m0 blocks (32 k each) per row: load bl stages block bl of 64 rows
-#pragma unroll
-      for (int bl = 0; bl < 2; ++bl)
-        s_voff[bl] = kw < p.K ? (int)(lane * p.ssn + (kw >> 5) + bl) : kOOB;
-    }
+  for (int rb = 0; rb < 2; ++rb)
+    b_voff[rb] = kw < p.K ? (int)((rb * 32 + (lane >> 1)) * p.sbn + kw / 2) + (lane & 1) * 16 : kOOB;
+  if constexpr (FMT == kNF4) {
+    s_voff[0] = kw < p.K ? (int)(lane * p.ssn * 4 + (kw >> 6) * 4) : kOOB;
+    s_voff[1] = kOOB;
   } else {
-    // loading lane i: row 32 rb + i / 2 of the wave's 64, 16-byte half i % 2
-    // (two lanes per row keep each lane quad on two cache lines); NF4
-    // scales: row i, one load; MXFP4 scales: row 32 rb + i / 2, block i % 2
+    // two e8m0 blocks (32 k each) per row: load bl stages block bl of 64 rows
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const int64_t n = t.n0 + wave * 64 + rb * 32 + (lane >> 1);
-      b_voff[rb] = n < p.N ? (int)(n * p.sbn) + (lane & 1) * 16 : kOOB;
-      if constexpr (FMT != kNF4) s_voff[rb] = n < p.N ? (int)(n * p.ssn) + (lane & 1) : kOOB;
-    }
-    if constexpr (FMT == kNF4) {
-      const int64_t n = t.n0 + wave * 64 + lane;
-      s_voff[0] = n < p.N ? (int)(n * p.ssn * 4) : kOOB;
-      s_voff[1] = kOOB;
-    }
+    for (int bl = 0; bl < 2; ++bl)
+      s_voff[bl] = kw < p.K ? (int)(lane * p.ssn + (kw >> 5) + bl) : kOOB;
   }
   // this wave's blocks of a weight slot: bytes (rb) at +rb KiB, lane-linear;
   // scales one dword per lane (direct-to-LDS loads of a byte still land in
@@ -2146,31 +2125,7 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   auto issue_w = [&](int g, int q0, int q1) {
     const bool live = g < F;
     const int k0 = live ? g * kPfBK : 0;
-    if constexpr (DG) {
-      // rows [k0, k0 + 64) of the contraction: 2 KiB of bytes, 64 scales
-      const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-          uniform_ptr(b_base), 0, uniform(live ? b_bytes : 0), 0x00020000);
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          uniform_ptr(s_base), 0, uniform(live ? s_bytes : 0), 0x00020000);
-      char* slot = smem + kPwW0 + uniform((g % 3) * kPwWSlot);
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-        if (b >= q0 && b < q1)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(slot + w_wave + b * 1024), 16,
-                                                   b_voff[b], uniform((int)(k0 * p.sbn)), 0, 0);
-      if constexpr (FMT == kNF4) {
-        if (2 >= q0 && 2 < q1)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(slot + s_wave), 4, s_voff[0],
-                                                   uniform((int)(k0 * p.ssn * 4)), 0, 0);
-      } else {
-#pragma unroll
-        for (int bl = 0; bl < 2; ++bl)
-          if (bl + 2 >= q0 && bl + 2 < q1)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(slot + s_wave + bl * 256), 1,
-                                                     s_voff[bl], uniform((int)(k0 * p.ssn)), 0, 0);
-      }
-      return;
-    }
+    // rows [k0, k0 + 64) of the contraction: 2 KiB of bytes, 64 scales
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
         uniform_ptr(b_base), 0, uniform(live ? b_bytes : 0), 0x00020000);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -2180,47 +2135,33 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
     for (int b = 0; b < 2; ++b)
       if (b >= q0 && b < q1)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(slot + w_wave + b * 1024), 16,
-                                                 b_voff[b], uniform(k0 >> 1), 0, 0);
+                                                 b_voff[b], uniform((int)(k0 * p.sbn)), 0, 0);
     if constexpr (FMT == kNF4) {
       if (2 >= q0 && 2 < q1)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(slot + s_wave), 4, s_voff[0],
-                                                 uniform((k0 >> 6) * 4), 0, 0);
+                                                 uniform((int)(k0 * p.ssn * 4)), 0, 0);
     } else {
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        if (b + 2 < q0 || b + 2 >= q1) continue;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(slot + s_wave + b * 256), 1,
-                                                 s_voff[b], uniform(k0 >> 5), 0, 0);
-      }
+      for (int bl = 0; bl < 2; ++bl)
+        if (bl + 2 >= q0 && bl + 2 < q1)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(slot + s_wave + bl * 256), 1,
+                                                   s_voff[bl], uniform((int)(k0 * p.ssn)), 0, 0);
     }
   };
-  // this lane's packed bytes and scale of step g (block rb), from its slot
-  // dgrad: lane address of the tr8 read of slice kk (lane i of its 16-lane
+  // lane address of the tr8 read of slice kk (lane i of its 16-lane
   // group supplies 8 bytes of row pi(i / 2), half i % 2 of the group's 16)
   const int tr_off = w_wave + (32 * h + ((lane >> 1) & 3) * 2 + ((lane >> 3) & 1)) * 32 +
                      ((lane >> 4) & 1) * 16 + (lane & 1) * 8;
-  auto read_w = [&](int g, u32x4_t (&w)[2], float (&sc)[2]) {
+  // this lane's packed bytes of step g, from its slot
+  auto read_w = [&](int g, u32x4_t (&w)[2]) {
     const char* slot = smem + kPwW0 + uniform((g % 3) * kPwWSlot);
-    if constexpr (DG) {
-      typedef __attribute__((address_space(3))) v2i32_t lds_v2i32;
+    typedef __attribute__((address_space(3))) v2i32_t lds_v2i32;
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const v2i32_t r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-            (lds_v2i32*)(lds_ptr_t)(slot + tr_off + kk * 8 * 32));
-        w[0][kk] = (unsigned)r.x;
-        w[1][kk] = (unsigned)r.y;
-      }
-      sc[0] = sc[1] = 0.f;
-      return;
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      w[b] = *reinterpret_cast<const u32x4_t*>(slot + w_wave + b * 1024 + (2 * l32 + h) * 16);
-      if constexpr (FMT == kNF4)
-        sc[b] = *reinterpret_cast<const float*>(slot + s_wave + (b * 32 + l32) * 4);
-      else
-        sc[b] = e8m0_to_f32(
-            *reinterpret_cast<const uint8_t*>(slot + s_wave + b * 256 + (2 * l32 + h) * 4));
+    for (int kk = 0; kk < 4; ++kk) {
+      const v2i32_t r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (lds_v2i32*)(lds_ptr_t)(slot + tr_off + kk * 8 * 32));
+      w[0][kk] = (unsigned)r.x;
+      w[1][kk] = (unsigned)r.y;
     }
   };
 
@@ -2232,59 +2173,47 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   // MFMAs. Parity q alternates between targets.
   float2 tp[2][2][4];   // NF4: table pairs [q][rb][byte of the dword]
   unsigned traw[2][2];  // MXFP4: the packed dword [q][rb]
-  float ts[2][2];       // the target's scale [q][rb]
-  float ts8[2][DG ? 8 : 1];   // dgrad: the scales of the target's 8 rows [q][row]
+  float ts8[2][8];      // the scales of the target's 8 rows [q][row]
   // Both phases come in 8 pieces (pc), so the slice loop can spread them
   // over its MFMA pairs.
-  // Lookup piece pc: NF4 table pair of byte pc % 4 of dword pc / 4 (dgrad:
-  // piece 0 also reads the target rows' 8 scales); MXFP4 keeps dword pc.
-  // (dgrad) g, kk: the target's step and slice, whose rows' scales it reads
-  auto lookup_pc = [&](auto QI, unsigned x0, unsigned x1, const float (&sc)[2], int g, int kk,
-                       int pc) {
+  // Lookup piece pc: NF4 table pair of byte pc % 4 of dword pc / 4; MXFP4 keeps
+  // dword pc. Piece 0 also reads the scales of the target's (step g, slice
+  // kk) 8 rows.
+  auto lookup_pc = [&](auto QI, unsigned x0, unsigned x1, int g, int kk, int pc) {
     constexpr int q = decltype(QI)::value;
-    const int b = pc >> 2, i = pc & 3;
-    const unsigned xb = b ? x1 : x0;
-    if constexpr (DG) {
-      if (pc == 0) {
-        // MXFP4: the lane's byte column c = lane % 32 holds k = 2c, 2c + 1,
-        // in scale block c / 16; each staged byte sits in its own dword
-        const char* sp = smem + kPwW0 + uniform((g % 3) * kPwWSlot) + s_wave + (32 * h + 8 * kk) * 4 +
-                         (FMT == kNF4 ? 0 : (l32 >> 4) * 256);
-        const u32x4_t s0 = *reinterpret_cast<const u32x4_t*>(sp);
-        const u32x4_t s1 = *reinterpret_cast<const u32x4_t*>(sp + 16);
+    if (pc == 0) {
+      // MXFP4: the lane's byte column c = lane % 32 holds k = 2c, 2c + 1,
+      // in scale block c / 16; each staged byte sits in its own dword
+      const char* sp = smem + kPwW0 + uniform((g % 3) * kPwWSlot) + s_wave + (32 * h + 8 * kk) * 4 +
+                       (FMT == kNF4 ? 0 : (l32 >> 4) * 256);
+      const u32x4_t s0 = *reinterpret_cast<const u32x4_t*>(sp);
+      const u32x4_t s1 = *reinterpret_cast<const u32x4_t*>(sp + 16);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if constexpr (FMT == kNF4) {
-            ts8[q][r] = __uint_as_float(s0[r]);
-            ts8[q][4 + r] = __uint_as_float(s1[r]);
-          } else {
-            ts8[q][r] = e8m0_to_f32(s0[r] & 0xFFu);
-            ts8[q][4 + r] = e8m0_to_f32(s1[r] & 0xFFu);
-          }
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (FMT == kNF4) {
+          ts8[q][r] = __uint_as_float(s0[r]);
+          ts8[q][4 + r] = __uint_as_float(s1[r]);
+        } else {
+          ts8[q][r] = e8m0_to_f32(s0[r] & 0xFFu);
+          ts8[q][4 + r] = e8m0_to_f32(s1[r] & 0xFFu);
         }
-      }
-      if constexpr (FMT != kNF4) {
-        if (pc < 2) traw[q][pc] = pc ? x1 : x0;
-        return;
       }
     }
     if constexpr (FMT == kNF4) {
-      if (i == 0) ts[q][b] = sc[b];
-      unsigned addr = __builtin_amdgcn_perm(xb, reg2, 0x0C020000u | ((4u + i) << 8)) >> 1;
+      const int b = pc >> 2, i = pc & 3;
+      const unsigned addr =
+          __builtin_amdgcn_perm(b ? x1 : x0, reg2, 0x0C020000u | ((4u + i) << 8)) >> 1;
       tp[q][b][i] = *reinterpret_cast<const float2*>(smem + addr);
     } else {
-      if (pc < 2) {
-        traw[q][pc] = pc ? x1 : x0;
-        ts[q][pc] = sc[pc];
-      }
+      if (pc < 2) traw[q][pc] = pc ? x1 : x0;
     }
   };
-  // Math piece pc: one bf16-pair dword of operand block pc / 4, dword pc % 4
-  // (dgrad: dword pc / 2 of block pc % 2); MXFP4 converts block pc whole.
+  // Math piece pc: bf16-pair dword pc / 2 of operand block pc % 2 (MXFP4: of
+  // both blocks, in the even pieces).
   auto math_pc = [&](auto QI, auto DI, int pc) {
     constexpr int q = decltype(QI)::value;
     constexpr int d = decltype(DI)::value;
-    if constexpr (DG && FMT != kNF4) {
+    if constexpr (FMT != kNF4) {
       // byte m of dword 0 / 1: rows 2m / 2m + 1, low nibble even k; the
       // convert applies each row's own scale, a byte permute pairs the rows
       if (pc & 1) return;
@@ -2301,23 +2230,18 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
       const unsigned c1 = cvt(traw[q][1], ts8[q][2 * m + 1]);
       wf[0][d][m] = __builtin_amdgcn_perm(c1, c0, 0x05040100u);
       wf[1][d][m] = __builtin_amdgcn_perm(c1, c0, 0x07060302u);
-    } else if constexpr (DG) {
+    } else {
       // byte m of dword 0 / 1: rows 2m / 2m + 1; .x even k, .y odd k
       const int m = pc >> 1;
       if (pc & 1)
         wf[1][d][m] = bf16x2_bits(tp[q][0][m].y * ts8[q][2 * m], tp[q][1][m].y * ts8[q][2 * m + 1]);
       else
         wf[0][d][m] = bf16x2_bits(tp[q][0][m].x * ts8[q][2 * m], tp[q][1][m].x * ts8[q][2 * m + 1]);
-    } else if constexpr (FMT == kNF4) {
-      const int b = pc >> 2, i = pc & 3;
-      wf[b][d][i] = bf16x2_bits(tp[q][b][i].x * ts[q][b], tp[q][b][i].y * ts[q][b]);
-    } else {
-      if (pc < 2) wf[pc][d] = mx_dword_to_bf16(traw[q][pc], ts[q][pc]);
     }
   };
-  auto lookup = [&](auto QI, unsigned x0, unsigned x1, const float (&sc)[2], int g, int kk) {
+  auto lookup = [&](auto QI, unsigned x0, unsigned x1, int g, int kk) {
 #pragma unroll
-    for (int pc = 0; pc < 8; ++pc) lookup_pc(QI, x0, x1, sc, g, kk, pc);
+    for (int pc = 0; pc < 8; ++pc) lookup_pc(QI, x0, x1, g, kk, pc);
   };
   auto math = [&](auto QI, auto DI) {
 #pragma unroll
@@ -2355,16 +2279,15 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   __builtin_amdgcn_s_barrier();
   issue_a(2, 0, 3);   // the rest of this group goes out during step 0
   u32x4_t wn[2];
-  float sn[2];
-  read_w(0, wn, sn);
-  lookup(I1{}, wn[0][0], wn[1][0], sn, 0, 0);
+  read_w(0, wn);
+  lookup(I1{}, wn[0][0], wn[1][0], 0, 0);
   math(I1{}, I0{});
-  lookup(I1{}, wn[0][1], wn[1][1], sn, 0, 1);
+  lookup(I1{}, wn[0][1], wn[1][1], 0, 1);
   math(I1{}, I1{});
-  lookup(I1{}, wn[0][2], wn[1][2], sn, 0, 2);
+  lookup(I1{}, wn[0][2], wn[1][2], 0, 2);
   math(I1{}, I2{});
-  lookup(I0{}, wn[0][3], wn[1][3], sn, 0, 3);   // step 0's slice 3, decoded during its slice 0
-  read_w(1, wn, sn);
+  lookup(I0{}, wn[0][3], wn[1][3], 0, 3);   // step 0's slice 3, decoded during its slice 0
+  read_w(1, wn);
   u32x4_t av[kM];
 #pragma unroll
   for (int i = 0; i < kM; ++i)
@@ -2374,8 +2297,6 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int i = 0; i < kM; ++i) acc[b][i] = f32x16_t{};
-
-  // instruction mix of one slice, for the interleaving below
 
   for (int f = 0; f < F; ++f) {
     int ao[4];
@@ -2392,14 +2313,13 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
       // this slice's lookup input: for slice 3 it is saved before step
       // f + 2's bytes replace wn
       unsigned x0 = wn[0][kk], x1 = wn[1][kk];
-      float xs[2] = {sn[0], sn[1]};
       if constexpr (kk == 3) {
         // step f + 1's stage and step f + 2's weights have landed, every
         // wave has read all of stage f: publish, and start refilling it
         wait_vm_lgkm0<kGroupLoads>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        read_w(f + 2, wn, sn);
+        read_w(f + 2, wn);
       }
       constexpr int qn = (kk + 1) & 1, qc = kk & 1;
       using QN = std::integral_constant<int, qn>;
@@ -2434,7 +2354,7 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
         }
 #pragma unroll
         for (int pc = (8 * i) / kM; pc < (8 * (i + 1)) / kM; ++pc) {
-          lookup_pc(QN{}, x0, x1, xs, f + 1, kk, pc);
+          lookup_pc(QN{}, x0, x1, f + 1, kk, pc);
           math_pc(QC{}, DT{}, pc);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -2455,72 +2375,44 @@ __device__ __forceinline__ void prefill_w_tile(const FwdArgs& p, const PfTile t,
   __builtin_amdgcn_sched_barrier(0);
   wait_vm_lgkm0<0>();
   __builtin_amdgcn_s_barrier();
-  if constexpr (DG) {
-    // MFMA row 8 g + 4 h + q of block b is column 64 w + 2 (8 g + 4 h + q) + b:
-    // the two blocks interleave into one 16-byte chunk 8 w + 2 g + h
+  // MFMA row 8 g + 4 h + q of block b is column 64 w + 2 (8 g + 4 h + q) + b:
+  // the two blocks interleave into one 16-byte chunk 8 w + 2 g + h
 #pragma unroll
-    for (int i = 0; i < kM; ++i)
+  for (int i = 0; i < kM; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int row = i * 32 + l32;
-        const int chunk = wave * 8 + 2 * g + h;
-        u32x4_t v;
+    for (int g = 0; g < 4; ++g) {
+      const int row = i * 32 + l32;
+      const int chunk = wave * 8 + 2 * g + h;
+      u32x4_t v;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = bf16x2_bits(acc[0][i][4 * g + q], acc[1][i][4 * g + q]);
-        *reinterpret_cast<u32x4_t*>(smem + row * 512 + ((chunk ^ l32) << 4)) = v;
-      }
-  } else
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int i = 0; i < kM; ++i)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int row = i * 32 + l32;
-        const int col = wave * 64 + b * 32 + 8 * g + 4 * h;   // 4 columns
-        u32x2_t v;
-        v.x = bf16x2_bits(acc[b][i][4 * g + 0], acc[b][i][4 * g + 1]);
-        v.y = bf16x2_bits(acc[b][i][4 * g + 2], acc[b][i][4 * g + 3]);
-        *reinterpret_cast<u32x2_t*>(smem + row * 512 + (((col >> 3) ^ l32) << 4) + (col & 7) * 2) = v;
-      }
+      for (int q = 0; q < 4; ++q) v[q] = bf16x2_bits(acc[0][i][4 * g + q], acc[1][i][4 * g + q]);
+      *reinterpret_cast<u32x4_t*>(smem + row * 512 + ((chunk ^ l32) << 4)) = v;
+    }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(out + (int64_t)t.row0 * p.ldo), 0, uniform((int)((int64_t)t.rows * p.ldo * 2)),
       0x00020000);
   const int ldo2 = (int)(p.ldo * 2);
-  // whole 8-column chunks store 16 bytes; the chunk that straddles the
-  // output width (width % 8 == 4) stores its first 8 bytes only, so no
-  // store reaches past a row's last column. The stores are non-temporal
-  // (nt): the output is not read again here, and every CU reaches its
-  // epilogue at about the same time, so a tile's 128 KiB would otherwise
-  // push the next tiles' weights and activations out of L2 (down
-  // projection at M = 256: 760 -> 813 TFLOP/s).
+  // The stores are non-temporal (nt): the output is not read again here, and
+  // every CU reaches its epilogue at about the same time, so a tile's 128 KiB
+  // would otherwise push the next tiles' weights and gradients out of L2.
   const int chunk = lane & 31;
   const int col = t.n0 + chunk * 8;
-  const int coff16 = col + 8 <= Nout ? col * 2 + h * ldo2 : kOOB;
-  const int coff8 = col < Nout && col + 8 > Nout ? col * 2 + h * ldo2 : kOOB;
-  const bool straddle = Nout % 8 != 0;
-  // wave w stores rows 2 (4 j + w) + lane / 32, j = 0 .. 4 kM - 1
+  const int coff = col < p.K ? col * 2 + h * ldo2 : kOOB;   // K % 64 == 0
+  // wave w stores rows 2 (4 j + w) + lane / 32, j = 0 .. 4 kM - 1 (no scalar
+  // offset: see store_b128)
 #pragma unroll
   for (int j = 0; j < kM * 4; ++j) {
     const int row = (j * 4 + wave) * 2 + h;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(smem + row * 512 + ((chunk ^ (row & 31)) << 4));
-    const int so = uniform((j * 4 + wave) * 2 * ldo2);
-    __builtin_amdgcn_raw_buffer_store_b128(v, ro, coff16, so, kNonTemporal);
-    if (straddle) {
-      u32x2_t v2;
-      v2.x = v[0];
-      v2.y = v[1];
-      __builtin_amdgcn_raw_buffer_store_b64(v2, ro, coff8, so, kNonTemporal);
-    }
+    __builtin_amdgcn_raw_buffer_store_b128(v, ro, coff + (j * 4 + wave) * 2 * ldo2, 0, kNonTemporal);
   }
 }
 
-
-template <int FMT, bool DG = false>
+template <int FMT>
 __global__ void __launch_bounds__(256, 1)
-    k_prefill_w(const FwdArgs p, const int32_t* __restrict__ t_row0,
+    k_dgrad_tall(const FwdArgs p, const int32_t* __restrict__ t_row0,
                 const int32_t* __restrict__ t_rows, const int32_t* __restrict__ t_group,
                 const int32_t* __restrict__ eids, uint16_t* __restrict__ out, const PwTiles tt) {
   __shared__ __attribute__((aligned(16))) char smem[kPwLds];
@@ -2530,7 +2422,7 @@ __global__ void __launch_bounds__(256, 1)
   // XCD x = blockIdx % 8 takes the x-th contiguous eighth of the tile list;
   // its workgroups walk that range with a stride of their count (tiles come
   // largest first, so each workgroup gets one tile of every size band)
-  const int n_tiles = (int)(((DG ? p.K : p.N) + kPfBN - 1) / kPfBN);
+  const int n_tiles = (int)((p.K + kPfBN - 1) / kPfBN);
   const int64_t total = (int64_t)p.n_mtiles * n_tiles;
   const int nx = gridDim.x >= 8 ? 8 : 1;
   const int x = (int)(blockIdx.x % nx), idx = (int)(blockIdx.x / nx);
@@ -2559,13 +2451,13 @@ __global__ void __launch_bounds__(256, 1)
     }
     // MFMAs for the tile's 32-row subtiles only
     switch ((t.rows + 31) >> 5) {
-      case 8: prefill_w_tile<FMT, 8, DG>(p, t, smem, out, lut, first); break;
-      case 7: prefill_w_tile<FMT, 7, DG>(p, t, smem, out, lut, first); break;
-      case 6: prefill_w_tile<FMT, 6, DG>(p, t, smem, out, lut, first); break;
-      case 5: prefill_w_tile<FMT, 5, DG>(p, t, smem, out, lut, first); break;
-      case 4: prefill_w_tile<FMT, 4, DG>(p, t, smem, out, lut, first); break;
-      case 3: prefill_w_tile<FMT, 3, DG>(p, t, smem, out, lut, first); break;
-      default: prefill_w_tile<FMT, 2, DG>(p, t, smem, out, lut, first); break;
+      case 8: dgrad_tall_tile<FMT, 8>(p, t, smem, out, lut, first); break;
+      case 7: dgrad_tall_tile<FMT, 7>(p, t, smem, out, lut, first); break;
+      case 6: dgrad_tall_tile<FMT, 6>(p, t, smem, out, lut, first); break;
+      case 5: dgrad_tall_tile<FMT, 5>(p, t, smem, out, lut, first); break;
+      case 4: dgrad_tall_tile<FMT, 4>(p, t, smem, out, lut, first); break;
+      case 3: dgrad_tall_tile<FMT, 3>(p, t, smem, out, lut, first); break;
+      default: dgrad_tall_tile<FMT, 2>(p, t, smem, out, lut, first); break;
     }
     first = false;
   }
@@ -2574,7 +2466,7 @@ __global__ void __launch_bounds__(256, 1)
 // ========================================================== tiled dgrad ==
 //
 // out[t, k] = sum_n grad[t, n] W[e][n, k]: the weights are read transposed.
-// Same skeleton as k_prefill -- 128-row tiles of one group x 256 output
+// 128-row tiles of one group x 256 output
 // columns (here: k), a persistent XCD-contiguous tile list, a 4-stage ring of
 // gradient rows filled by direct-to-LDS loads, one flat pipeline over (tile,
 // 64-wide n-step) -- with the weight operand going through LDS:
@@ -3684,7 +3576,7 @@ const PwTiles& no_tiles() {
 // Workgroups per XCD range of the persistent tile grids: one per CU
 // (each walks several tiles; the pair table is built once per workgroup), or
 // fewer when the XCD's range has fewer tiles.
-int64_t prefill_w_per_xcd(int64_t tiles, int cus) {
+int64_t tiles_per_xcd(int64_t tiles, int cus) {
   const int64_t per_x = (tiles + 7) / 8;
   const int64_t cap = cus >= 8 ? cus / 8 : 1;
   return per_x > cap ? cap : per_x;
@@ -3707,7 +3599,7 @@ int launch_fwd(const FwdArgs& p, int block_m, hipStream_t stream, const PwTiles*
     if (tile_ok) {
       const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kPfBN - 1) / kPfBN);
       // the grid covers eight equal XCD ranges
-      const int64_t per_x = prefill_w_per_xcd(tiles, cus);
+      const int64_t per_x = tiles_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
       return launch_tile_fwd(FMT, p, tt ? *tt : no_tiles(), per_x, stream);
     }
@@ -3755,11 +3647,11 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
       f.ldo = p.ldo;
       const int64_t tiles = (int64_t)p.n_mtiles * ((p.K + kPfBN - 1) / kPfBN);
       const int64_t wide = (int64_t)p.n_mtiles * ((p.K + 2 * kPfBN - 1) / (2 * kPfBN));
-      const int64_t per_x = prefill_w_per_xcd(tiles, cus);
+      const int64_t per_x = tiles_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
       // Two kernels with the same bits. A 512-column tile of k_tile_dgrad
-      // takes 1.3 (32 rows) to 1.75 (128 rows) times a 256-column tile of
-      // k_prefill_w, and two such 1.45 to 2 times as long, so it is taken
+      // takes 1.3 (32 rows) to 1.8 (160 rows) times a 256-column tile of
+      // k_dgrad_tall, so it is taken
       // where it needs at most 5/9 of the rounds of tiles over the CUs
       // (128 experts, N = 2048, K = 768: 1 against 2 rounds, 75 against 89 us
       // at 128 rows); with fewer tiles than that, CUs would stand idle.
@@ -3770,9 +3662,9 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
         f.t_group = p.t_group;
         f.eids = p.eids;
         return launch_tile_dgrad(FMT, f, p.out, tt ? *tt : no_tiles(),
-                                 prefill_w_per_xcd(wide, cus), stream);
+                                 tiles_per_xcd(wide, cus), stream);
       }
-      hipLaunchKernelGGL((k_prefill_w<FMT, true>), dim3((unsigned)(per_x * 8)), dim3(256), 0, stream,
+      hipLaunchKernelGGL((k_dgrad_tall<FMT>), dim3((unsigned)(per_x * 8)), dim3(256), 0, stream,
                          f, p.t_row0, p.t_rows, p.t_group, p.eids, p.out, tt ? *tt : no_tiles());
       return hipGetLastError() == hipSuccess ? 0 : -2;
     }

@@ -1,6 +1,6 @@
 // gnf4_tile.hip -- the eight-wave tile kernels of the grouped 4-bit expert
 // GEMM on gfx950: the forward (up to 256 token rows of one group x 256 weight
-// rows per tile) and the dgrad of groups of up to 128 rows (k_tile_dgrad).
+// rows per tile) and the dgrad of groups of up to 160 rows (k_tile_dgrad).
 //
 // k_tile_fwd: eight waves (two per SIMD) on a persistent grid of one workgroup
 // per CU. Wave w owns 32 weight rows for all of the tile's token rows, so no
@@ -684,7 +684,7 @@ __global__ void __launch_bounds__(512, 2)
 
 // ================================================================ dgrad ==
 //
-// k_tile_dgrad: out[t, k] = sum_n grad[t, n] W[e][n, k], tiles of up to 128
+// k_tile_dgrad: out[t, k] = sum_n grad[t, n] W[e][n, k], tiles of up to 160
 // gradient rows of one group x 512 output columns (k), the contraction over n
 // in ascending steps of 64 packed rows. Eight waves, two per SIMD, of 64
 // columns each: no weight is decoded twice, and one wave's lookups run while
@@ -703,16 +703,18 @@ __global__ void __launch_bounds__(512, 2)
 //     them, each row by its own scale, in its second;
 //   * the loads run on into the workgroup's next tile.
 // The products of an output are added in the 256-row kernel's order: both
-// give the same bits.
+// give the same bits. 160 rows are what fits: the accumulators take 160 of a
+// wave's 256 registers, the rings and the table 148 KiB of LDS.
 // What bounds it: at 128 rows the MFMAs (1024 clocks per wave and step, 2048
 // per SIMD) and the LDS (lookups, operand reads and stage writes, about 2400
 // clocks) half hide each other, a step takes 3800-4500; at 32 rows the chain
 // of lookup, pack and MFMA.
-// Measured (MI355X, 32 / 64 / 128 rows per group; before: the 256-row
-// kernel): NF4, 128 experts, N = 2048, K = 768: 45 / 54 / 75 us (67 / 69 / 89);
-// N = 1536, K = 2048: 71 / 88 / 119 (105 / 110 / 147); MXFP4, 32 experts,
-// N = 5760, K = 2880: 99 / 116 / 163 (177 / 177 / 201). Two halves of the step
-// list per tile instead of two tiles' columns: 49 / 59 / 80, and other bits.
+// Measured (MI355X, 32 / 64 / 128 / 160 rows per group; before: the 256-row
+// kernel): NF4, 128 experts, N = 2048, K = 768: 45 / 54 / 73 / 83 us (67 / 69 /
+// 89 / 92); N = 1536, K = 2048: 74 / 88 / 118 / 135 (105 / 110 / 147 / 160);
+// MXFP4, 32 experts, N = 5760, K = 2880: 102 / 117 / 164 / 189 us (177 / 177 /
+// 201 / 222). Two waves per 64 columns, each with every second step: 49 / 59 /
+// 80 us at 32 / 64 / 128 rows of the first shape, and other bits.
 // A wave loading its own 32 bytes of every row: 133 us for MXFP4 at 32 rows.
 constexpr int kDtBM = kDgradWideRows;
 constexpr int kDtBN = 512;

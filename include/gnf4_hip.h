@@ -345,7 +345,8 @@ int gnf4_hip_nf4_ffn_noalloc_reset(uint32_t *error_word, void *stream);
  * ldo >= K. Tile table as for the forward tiled path (n_mtiles may be 0:
  * nothing to do). With N % 64 == 0 and K % 64 == 0 any block_m up to 256 is
  * taken by the persistent kernels that read the packed rows transposed (512
- * columns per tile for block_m <= 128 where enough tiles fill the device);
+ * columns per tile for block_m <= 128 where enough tiles fill the device, the
+ * same bits);
  * other shapes need block_m <= 128 (-1 otherwise). */
 int gnf4_hip_grouped_dgrad(int fmt, const void *grad_out, int g_dtype, int64_t ldg,
                            const uint8_t *B, int64_t stride_be, int64_t stride_bn,
