@@ -619,14 +619,21 @@ struct TileWalk {
     lo = total * x / nx;
     hi = total * (x + 1) / nx;
   }
-  // tile tg of the list; rows 0: none
-  __device__ __forceinline__ PfTile at(int64_t tg, const int32_t* __restrict__ t_row0,
-                                       const int32_t* __restrict__ t_rows,
-                                       const int32_t* __restrict__ t_group,
-                                       const int32_t* __restrict__ eids, const PwTiles& tt) const {
+  // The workgroup's first tile with rows from tg on; tg advances to it. A
+  // device table may hold empty tiles anywhere (a kernel-argument table does
+  // not): they are stepped over. Rows 0: the list has ended.
+  __device__ __forceinline__ PfTile next(int64_t& tg, const int32_t* __restrict__ t_row0,
+                                         const int32_t* __restrict__ t_rows,
+                                         const int32_t* __restrict__ t_group,
+                                         const int32_t* __restrict__ eids, const PwTiles& tt) const {
     PfTile t{0, 0, 0, 0};
+    int mt = (int)(tg / n_tiles);
+    if (tt.n == 0)
+      while (tg < hi && t_rows[mt] <= 0) {
+        tg += stride;
+        mt = (int)(tg / n_tiles);
+      }
     if (tg >= hi) return t;
-    const int mt = (int)(tg / n_tiles);
     t.n0 = uniform((int)(tg - (int64_t)mt * n_tiles) * width);
     if (tt.n > 0) {
       t.row0 = uniform(tt.row0[mt]);
@@ -649,7 +656,7 @@ __global__ void __launch_bounds__(512, 2)
   __shared__ __attribute__((aligned(16))) char smem[kTlLds];
   const TileWalk tw(p, kTlBN, (int)((p.N + kTlBN - 1) / kTlBN));
   int64_t tg = tw.lo + tw.idx;
-  PfTile t = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+  PfTile t = tw.next(tg, t_row0, t_rows, t_group, eids, tt);
   if (t.rows <= 0) return;
   const int F = uniform((int)(p.K / kTlBK));
   TileRegs<FMT> regs;
@@ -664,7 +671,7 @@ __global__ void __launch_bounds__(512, 2)
   int slot = 0;
   while (t.rows > 0) {
     tg += tw.stride;
-    const PfTile tn = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+    const PfTile tn = tw.next(tg, t_row0, t_rows, t_group, eids, tt);
     switch ((t.rows + 31) >> 5) {
       case 8: slot = tile_fwd<FMT, 8>(p, t, tn, smem, out, regs, slot); break;
       case 7: slot = tile_fwd<FMT, 7>(p, t, tn, smem, out, regs, slot); break;
@@ -1048,7 +1055,7 @@ __global__ void __launch_bounds__(512, 2)
   __shared__ __attribute__((aligned(16))) char smem[kTlLds];
   const TileWalk tw(p, kDtBN, (int)((p.K + kDtBN - 1) / kDtBN));
   int64_t tg = tw.lo + tw.idx;
-  PfTile t = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+  PfTile t = tw.next(tg, t_row0, t_rows, t_group, eids, tt);
   if (t.rows <= 0) return;
   {
     const int lane = opaque(threadIdx.x) & 63, wave = uniform(threadIdx.x >> 6);
@@ -1068,7 +1075,7 @@ __global__ void __launch_bounds__(512, 2)
   DgradPos at{0, 0};
   while (t.rows > 0) {
     tg += tw.stride;
-    const PfTile tn = tw.at(tg, t_row0, t_rows, t_group, eids, tt);
+    const PfTile tn = tw.next(tg, t_row0, t_rows, t_group, eids, tt);
     switch ((t.rows + 31) >> 5) {
       case 5: at = tile_dgrad<FMT, 5>(p, t, tn, smem, out, at); break;
       case 4: at = tile_dgrad<FMT, 4>(p, t, tn, smem, out, at); break;

@@ -34,7 +34,8 @@
  *   n_mtiles  > 0 -> tiled path: the tile table t_row0/t_rows/t_group
  *                    [n_mtiles] int32 (reference build_group_tiles,
  *                    kernel/nf4_grouped.py:334-362) with block_m in
- *                    {16, 32, 64, 128, 256}; t_rows[i] <= block_m. With
+ *                    {16, 32, 64, 128, 256}; t_rows[i] <= block_m (entries
+ *                    of 0 rows may stand anywhere: nothing to do). With
  *                    K % 64 == 0, N % 4 == 0, ldo % 4 == 0 and an 8-byte
  *                    aligned out every height runs the eight-wave tile
  *                    kernel; 256 needs them (-1 otherwise). The order is free

@@ -11,7 +11,7 @@ come out bit for bit."""
 import pytest
 import torch
 
-from _fixtures import fp64_ref, rand_acts, rel_err
+from _fixtures import dequant, fp64_ref, rand_acts, rel_err
 from test_gpu_forward import _ops, _stack
 
 pytestmark = pytest.mark.gpu
@@ -59,3 +59,55 @@ def test_many_tiles_per_workgroup(fmt, K, mix):
     sizes = torch.randint(lo, hi + 1, (E,), generator=g).tolist()
     W, S = _stack(fmt, E, 1540, K, seed=K + 1)
     _check(fmt, W, S, sizes, torch.randperm(E, generator=g).tolist(), K, heights=(128,))
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
+@pytest.mark.parametrize("kind,bm,K", [("fwd", 256, 320), ("dgrad", 256, 576), ("dgrad", 128, 1024)])
+@pytest.mark.parametrize("empty", ["some", "first_and_last", "all"])
+def test_empty_tiles_in_a_device_table(fmt, kind, bm, K, empty):
+    """A table of fixed capacity has entries of no rows, anywhere: nothing is
+    computed for them, and every other tile is written with the bits of the
+    table without them. 384 entries, several per workgroup; on 256 CUs the
+    dgrad calls reach both the 256-row and the 512-column kernel (K = 1024: 3
+    rounds of tiles against 6)."""
+    import _hiplib
+    n, N = 384, 128
+    g = torch.Generator().manual_seed(bm + K)
+    rows = torch.randint(1, min(bm, 160) + 1, (n,), generator=g)
+    if empty == "some":
+        rows[torch.rand(n, generator=g) < 0.4] = 0
+    elif empty == "first_and_last":
+        rows[:40] = 0
+        rows[-40:] = 0
+    else:
+        rows[:] = 0
+    W, S = _stack(fmt, 4, N, K, seed=7)
+    T = max(int(rows.sum()), 1)
+    x = rand_acts(T, K if kind == "fwd" else N, seed=8)
+    width = N if kind == "fwd" else K
+    row0 = torch.cumsum(rows, 0) - rows
+    call = getattr(_hiplib.load(), "gnf4_hip_grouped_" + kind)
+
+    def run(keep):
+        dev = lambda v: v.to(torch.int32).cuda()  # noqa: E731
+        eids, t0, tr = dev(torch.arange(n) % 4), dev(row0[keep]), dev(rows[keep])
+        tg = dev(torch.arange(n)[keep])
+        out = torch.full((T, width), 7.0, dtype=torch.bfloat16, device="cuda")
+        head = (0 if fmt == "nf4" else 1, x.data_ptr(), _hiplib.DTYPE_BF16, x.stride(0),
+                W.data_ptr(), W.stride(0), W.stride(1), S.data_ptr(), S.stride(0), S.stride(1),
+                eids.data_ptr())
+        mid = (None, n) if kind == "fwd" else ()
+        _hiplib.check(call(*head, *mid, t0.data_ptr(), tr.data_ptr(), tg.data_ptr(), t0.numel(),
+                           bm, N, K, out.data_ptr(), out.stride(0),
+                           torch.cuda.current_stream().cuda_stream), kind)
+        return out
+
+    got = run(torch.ones(n, dtype=torch.bool))
+    if empty == "all":
+        assert bool((got == 7).all())
+        return
+    assert torch.equal(got, run(rows > 0))
+    w = [dequant(fmt, W[e], S[e]).double() for e in range(4)]
+    ref = torch.cat([x[r0:r0 + m].double() @ (w[i % 4].t() if kind == "fwd" else w[i % 4])
+                     for i, (r0, m) in enumerate(zip(row0.tolist(), rows.tolist())) if m])
+    assert rel_err(got, ref) <= 1e-2
