@@ -255,6 +255,17 @@ class _LoraTables:
                 self.n)
 
 
+def _rows(t):
+    """``t [T, C]`` as the kernels read it: 16-byte aligned rows of unit stride
+    that do not overlap. Anything else is copied: a gradient may come
+    broadcast (row stride 0, from ``out.sum(0)``), transposed or at any
+    offset."""
+    if (t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1]
+            or t.data_ptr() % 16):
+        return t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
 def _lora_call(name, dev, *args):
     with nf4_grouped._device_ctx(dev):
         rc = getattr(_hiplib.load(), name)(*args, nf4_grouped._stream_ptr(dev))
@@ -294,13 +305,13 @@ class _LoraAdd(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, base, a_cat, lora_A, lora_B, sizes, expert_ids, scaling):
-        a = nf4_grouped._act_view(a_cat.detach())
+        a = _rows(a_cat.detach())
         tb = _LoraTables(sizes, expert_ids, a.device)
         u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
         ctx.save_for_backward(a_cat, lora_A, lora_B, u)
         ctx.tables, ctx.args = tb, (sizes, expert_ids, scaling)
         return _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling),
-                        nf4_grouped._act_view(base))
+                        _rows(base))
 
     @staticmethod
     def backward(ctx, g):
@@ -314,10 +325,10 @@ class _LoraAdd(torch.autograd.Function):
                 got = iter(torch.autograd.grad(d, ins, g, create_graph=True) if ins else ())
             return (g, *(next(got) if n else None for n in need[1:4]), None, None, None)
         tb, s = ctx.tables, float(scaling)
-        gv = nf4_grouped._act_view(g)
+        gv = _rows(g)
         gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
         ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None
-        gA = _lora_wgrad(nf4_grouped._act_view(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
+        gA = _lora_wgrad(_rows(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
         gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
         return g, ga, gA, gB, None, None, None
 

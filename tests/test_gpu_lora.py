@@ -102,3 +102,38 @@ def test_double_backward_and_saved_tensor_hooks(monkeypatch):
         ga, = torch.autograd.grad(out, a, go, create_graph=True)
         res.append(torch.autograd.grad(ga.square().sum(), b)[0])
     assert rel_err(res[0], res[1].double()) <= 1e-4
+
+
+@pytest.mark.parametrize("form,train_x", [
+    (f, x) for f in ("broadcast", "padded", "odd_pad", "transposed") for x in (True, False)
+] + [("offset", False)])
+def test_gradients_of_every_layout(form, train_x, monkeypatch):
+    """The incoming gradient in the layouts that autograd and callers produce:
+    broadcast over the rows (``out.sum(0)``), rows of a wider buffer with
+    aligned and odd strides, a transposed tensor, a dense one at an odd
+    offset (the base half's dgrad refuses that one, so the activations are
+    not trained there)."""
+    import nf4_qlora
+    sizes, ids, N = [9, 30, 1], [1, 0, 2], 64
+    W, S, x, A, B, go = _case(sizes, ids, 3, 128, N, 8)
+    T = sum(sizes)
+    if form == "broadcast":
+        g = go[0].expand(T, N)
+    elif form in ("padded", "odd_pad"):
+        g = torch.zeros(T, N + (16 if form == "padded" else 3), dtype=go.dtype, device="cuda")
+        g[:, :N] = go
+        g = g[:, :N]
+    elif form == "transposed":
+        g = go.t().contiguous().t()
+    else:
+        g = torch.empty(T * N + 1, dtype=go.dtype, device="cuda")[1:].view(T, N).copy_(go)
+    res = []
+    for kernels in (True, False):
+        if not kernels:
+            monkeypatch.setattr(nf4_qlora, "_kernels_take", lambda *a: False)
+        ins = [A.clone().requires_grad_(True), B.clone().requires_grad_(True)]
+        xt = x.clone().requires_grad_(train_x)
+        out = nf4_qlora.fused_grouped_lora(xt, W, S, sizes, ids, *ins, scaling=2.0)
+        res.append(torch.autograd.grad(out, ([xt] if train_x else []) + ins, g))
+    for a, b in zip(*res):
+        assert rel_err(a, b.double()) <= (1e-3 if a.dtype == torch.bfloat16 else 1e-5)
