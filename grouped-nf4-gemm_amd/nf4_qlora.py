@@ -214,10 +214,14 @@ def _transforming() -> bool:
             or torch.is_autocast_enabled())
 
 
-def _kernels_take(out, a_cat, lora_A, lora_B, sizes) -> bool:
+def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling) -> bool:
     """Whether the HIP kernels take this low-rank delta: bf16 rows and fp32
     adapters on one GPU, plain contiguous tensors, r % 4 == 0 and r <= 64,
-    widths that are multiples of 8, every row in a group."""
+    widths that are multiples of 8, every row in a group, and a plain number
+    as ``scaling`` (a tensor may be learnable, live on the device or have one
+    value per column: the torch composition multiplies by it)."""
+    if not isinstance(scaling, (int, float)):
+        return False
     ts = (out, a_cat, lora_A, lora_B)
     if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
                and t.device == out.device for t in ts):
@@ -342,7 +346,7 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
                                   weights_fn=weights_fn, dgrad_kernel=dgrad_kernel)
     if lora_A is None or lora_B is None:
         return out
-    if _kernels_take(out, a_cat, lora_A, lora_B, sizes):
+    if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling):
         return _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     delta = lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     return out if delta is None else out + delta.to(out.dtype)

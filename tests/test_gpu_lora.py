@@ -137,3 +137,22 @@ def test_gradients_of_every_layout(form, train_x, monkeypatch):
         res.append(torch.autograd.grad(out, ([xt] if train_x else []) + ins, g))
     for a, b in zip(*res):
         assert rel_err(a, b.double()) <= (1e-3 if a.dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("shape", [(), (64,)])
+def test_tensor_scaling_is_multiplied_and_learned(shape):
+    """A scaling that is a tensor (a learnable scalar, one factor per output
+    column) enters the product and receives its gradient."""
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, go = _case(sizes, ids, 2, 128, 64, 8)
+    s = torch.full(shape, 1.5, device="cuda", requires_grad=True)
+    out = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B, scaling=s)
+    grad, = torch.autograd.grad(out, s, go)
+    base = nf4_qlora.gemm_4bit_grouped_train(x, W, S, sizes, ids)
+    d = torch.cat([(x[r].float() @ A[e].t()) @ B[e].t()
+                   for e, r in ((1, slice(0, 9)), (0, slice(9, 39)))])
+    assert rel_err(out, base.double() + 1.5 * d.double()) <= 1e-2   # two bf16 roundings
+    assert rel_err(grad, (go.double() * d.double()).sum_to_size(shape)) <= 1e-4
+    plain = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B, scaling=1.5)
+    assert rel_err(out.detach(), plain.double()) <= 1e-3
