@@ -240,19 +240,24 @@ def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling) -> bool:
 
 
 class _LoraTables:
-    """Device tables of one routing: tile and row offsets, expert ids."""
+    """Device tables of one routing: tile and row offsets, expert ids. Nothing
+    of the caller's is kept: it may write the next layer's routing into the
+    same tensor or list before backward."""
 
     def __init__(self, sizes, expert_ids, dev):
-        m = np.asarray([int(v) for v in sizes], dtype=np.int32)
+        self.sizes = [int(v) for v in sizes]
+        m = np.asarray(self.sizes, dtype=np.int32)
         off = np.zeros((2, len(m) + 1), dtype=np.int32)
         np.cumsum((m + 15) // 16, out=off[0, 1:])
         np.cumsum(m, out=off[1, 1:])
-        ids = nf4_grouped._eids_device(expert_ids, dev)
-        host = [*off] + ([] if ids is not None else [nf4_grouped._np_ids(expert_ids)])
-        views = nf4_grouped.to_device_i32(host, dev)
+        on_dev = torch.is_tensor(expert_ids) and expert_ids.is_cuda
+        ids = [] if on_dev else [nf4_grouped._np_ids(expert_ids)]
+        views = nf4_grouped.to_device_i32([*off, *ids], dev)
         self.n, self.G = int(off[0, -1]), len(m)
         self.tile_off, self.row_off = views[:2]
-        self.ids = ids.contiguous() if ids is not None else views[2]
+        self.ids = (torch.empty(self.G, dtype=torch.int32, device=dev).copy_(expert_ids)
+                    if on_dev else views[2])
+        self.expert_ids = self.ids if on_dev else ids[0].tolist()   # for the composition
 
     def args(self):
         return (self.tile_off.data_ptr(), self.row_off.data_ptr(), self.ids.data_ptr(), self.G,
@@ -313,22 +318,22 @@ class _LoraAdd(torch.autograd.Function):
         tb = _LoraTables(sizes, expert_ids, a.device)
         u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
         ctx.save_for_backward(a_cat, lora_A, lora_B, u)
-        ctx.tables, ctx.args = tb, (sizes, expert_ids, scaling)
+        ctx.tables, ctx.scaling = tb, scaling
         return _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling),
                         _rows(base))
 
     @staticmethod
     def backward(ctx, g):
         a_cat, A, B, u = ctx.saved_tensors
-        sizes, expert_ids, scaling = ctx.args
-        need = ctx.needs_input_grad
+        tb, scaling, need = ctx.tables, ctx.scaling, ctx.needs_input_grad
         if torch.is_grad_enabled():
             with torch.enable_grad():
                 ins = [t for t, n in zip((a_cat, A, B), need[1:4]) if n]
-                d = lora_delta_grouped(a_cat, A, B, sizes, expert_ids, scaling).to(g.dtype)
+                d = lora_delta_grouped(a_cat, A, B, tb.sizes, tb.expert_ids,
+                                       scaling).to(g.dtype)
                 got = iter(torch.autograd.grad(d, ins, g, create_graph=True) if ins else ())
             return (g, *(next(got) if n else None for n in need[1:4]), None, None, None)
-        tb, s = ctx.tables, float(scaling)
+        s = float(scaling)
         gv = _rows(g)
         gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
         ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None

@@ -156,3 +156,30 @@ def test_tensor_scaling_is_multiplied_and_learned(shape):
     assert rel_err(grad, (go.double() * d.double()).sum_to_size(shape)) <= 1e-4
     plain = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B, scaling=1.5)
     assert rel_err(out.detach(), plain.double()) <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64, None])
+@pytest.mark.parametrize("twice", [False, True])
+def test_routing_written_over_before_backward(dtype, twice, monkeypatch):
+    """A caller may reuse its routing buffers (a device tensor of either width,
+    host lists) for the next layer before this one's backward; ``twice``: also
+    before a gradient of the gradient."""
+    import nf4_qlora
+    W, S, x, A, B, go = _case([9, 30, 5], [1, 0, 2], 3, 128, 64, 8)
+    res = []
+    for kernels in (True, False):
+        if not kernels:
+            monkeypatch.setattr(nf4_qlora, "_kernels_take", lambda *a: False)
+        a, b = A.clone().requires_grad_(True), B.clone().requires_grad_(True)
+        sizes, ids = [9, 30, 5], [1, 0, 2]
+        if dtype is not None:
+            ids = torch.tensor(ids, dtype=dtype, device="cuda")
+        out = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, a, b, scaling=2.0)
+        if kernels:
+            sizes[:], ids[:] = [30, 5, 9], ([2, 2, 0] if dtype is None else 2)
+        grads = torch.autograd.grad(out, (a, b), go, create_graph=twice)
+        if twice:
+            grads = torch.autograd.grad(grads[0].square().sum() + grads[1].square().sum(), (a, b))
+        res.append(grads)
+    for p, q in zip(*res):
+        assert rel_err(p, q.double()) <= (1e-4 if twice else 1e-5)
