@@ -310,20 +310,37 @@ class _LoraAdd(torch.autograd.Function):
     """``base + bf16(scaling * (a A[e]^T) B[e]^T)`` through the kernels of
     csrc/gnf4_lora.hip (two forward, four backward launches, fp32 sums): the
     values and gradients of adding ``lora_delta_grouped``. A backward that is
-    itself differentiated runs that torch composition instead."""
+    itself differentiated runs that torch composition instead.
+
+    Backward reads copies of the activations and adapters, as the
+    composition's gathered ones are: a program may update the adapters, or
+    refill its activation buffer, before it. They are outputs of this function
+    as well, so that a second differentiation reaches the inputs through them
+    (MI355X, 8192 rows, 128 experts, K = 2048, N = 1536, r = 16: 26 of the
+    352 us of kernels of a training pass)."""
 
     @staticmethod
     def forward(ctx, base, a_cat, lora_A, lora_B, sizes, expert_ids, scaling):
+        need = ctx.needs_input_grad[1:4]
+        if any(need):
+            a_cat, lora_A, lora_B = a_cat.clone(), lora_A.clone(), lora_B.clone()
         a = _rows(a_cat.detach())
         tb = _LoraTables(sizes, expert_ids, a.device)
         u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
+        out = _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling), _rows(base))
+        if not any(need):
+            return out
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(a_cat, lora_A, lora_B, u)
         ctx.tables, ctx.scaling = tb, scaling
-        return _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling),
-                        _rows(base))
+        copies = (a_cat, lora_A, lora_B)
+        ctx.mark_non_differentiable(*(t for t, n in zip(copies, need) if not n))
+        return (out, *copies)
 
     @staticmethod
-    def backward(ctx, g):
+    def backward(ctx, g, *g_copies):
+        if g is None or not g_copies:
+            return (g, *(g_copies or (None,) * 3), None, None, None)
         a_cat, A, B, u = ctx.saved_tensors
         tb, scaling, need = ctx.tables, ctx.scaling, ctx.needs_input_grad
         if torch.is_grad_enabled():
@@ -331,15 +348,18 @@ class _LoraAdd(torch.autograd.Function):
                 ins = [t for t, n in zip((a_cat, A, B), need[1:4]) if n]
                 d = lora_delta_grouped(a_cat, A, B, tb.sizes, tb.expert_ids,
                                        scaling).to(g.dtype)
-                got = iter(torch.autograd.grad(d, ins, g, create_graph=True) if ins else ())
-            return (g, *(next(got) if n else None for n in need[1:4]), None, None, None)
-        s = float(scaling)
-        gv = _rows(g)
-        gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
-        ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None
-        gA = _lora_wgrad(_rows(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
-        gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
-        return g, ga, gA, gB, None, None, None
+                got = iter(torch.autograd.grad(d, ins, g, create_graph=True))
+            grads = [next(got) if n else None for n in need[1:4]]
+        else:
+            s = float(scaling)
+            gv = _rows(g)
+            gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
+            ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None
+            gA = _lora_wgrad(_rows(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
+            gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
+            grads = [ga, gA, gB]
+        grads = [x if y is None else y if x is None else x + y for x, y in zip(grads, g_copies)]
+        return (g, *grads, None, None, None)
 
 
 def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lora_B=None,
@@ -352,6 +372,7 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
     if lora_A is None or lora_B is None:
         return out
     if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling):
-        return _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
+        out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
+        return out[0] if isinstance(out, tuple) else out
     delta = lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     return out if delta is None else out + delta.to(out.dtype)

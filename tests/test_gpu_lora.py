@@ -183,3 +183,28 @@ def test_routing_written_over_before_backward(dtype, twice, monkeypatch):
         res.append(grads)
     for p, q in zip(*res):
         assert rel_err(p, q.double()) <= (1e-4 if twice else 1e-5)
+
+
+@pytest.mark.parametrize("train_x", [True, False])
+@pytest.mark.parametrize("twice", [False, True])
+def test_inputs_updated_in_place_before_backward(train_x, twice):
+    """An adapter update or a refilled activation buffer between forward and
+    backward changes no gradient and raises nothing."""
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, go = _case(sizes, ids, 2, 128, 64, 8)
+    res = []
+    for update in (False, True):
+        a, b = A.clone().requires_grad_(True), B.clone().requires_grad_(True)
+        xt = x.clone().requires_grad_(train_x)
+        ins = ([xt] if train_x else []) + [a, b]
+        out = nf4_qlora.fused_grouped_lora(xt, W, S, sizes, ids, a, b, scaling=2.0)
+        if update:
+            with torch.no_grad():
+                for t in (xt, a, b):
+                    t.mul_(3).add_(1)
+        grads = torch.autograd.grad(out, (a, b) if twice else ins, go, create_graph=twice)
+        if twice:
+            grads = torch.autograd.grad(sum(v.square().sum() for v in grads), (a, b))
+        res.append(grads)
+    assert all(torch.equal(p, q) for p, q in zip(*res))
