@@ -320,15 +320,16 @@ class _LoraAdd(torch.autograd.Function):
     352 us of kernels of a training pass)."""
 
     @staticmethod
-    def forward(ctx, base, a_cat, lora_A, lora_B, sizes, expert_ids, scaling):
-        need = ctx.needs_input_grad[1:4]
-        if any(need):
+    def forward(ctx, base, a_cat, lora_A, lora_B, sizes, expert_ids, scaling, recording):
+        need = ctx.needs_input_grad[1:4]   # by requires_grad, also under no_grad
+        recording = recording and any(need)
+        if recording:
             a_cat, lora_A, lora_B = a_cat.clone(), lora_A.clone(), lora_B.clone()
         a = _rows(a_cat.detach())
         tb = _LoraTables(sizes, expert_ids, a.device)
         u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
         out = _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling), _rows(base))
-        if not any(need):
+        if not recording:
             return out
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(a_cat, lora_A, lora_B, u)
@@ -340,7 +341,7 @@ class _LoraAdd(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g, *g_copies):
         if g is None or not g_copies:
-            return (g, *(g_copies or (None,) * 3), None, None, None)
+            return (g, *(g_copies or (None,) * 3), None, None, None, None)
         a_cat, A, B, u = ctx.saved_tensors
         tb, scaling, need = ctx.tables, ctx.scaling, ctx.needs_input_grad
         if torch.is_grad_enabled():
@@ -359,7 +360,7 @@ class _LoraAdd(torch.autograd.Function):
             gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
             grads = [ga, gA, gB]
         grads = [x if y is None else y if x is None else x + y for x, y in zip(grads, g_copies)]
-        return (g, *grads, None, None, None)
+        return (g, *grads, None, None, None, None)
 
 
 def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lora_B=None,
@@ -372,7 +373,8 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
     if lora_A is None or lora_B is None:
         return out
     if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling):
-        out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
+        out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling,
+                             torch.is_grad_enabled())
         return out[0] if isinstance(out, tuple) else out
     delta = lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling)
     return out if delta is None else out + delta.to(out.dtype)

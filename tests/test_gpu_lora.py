@@ -208,3 +208,19 @@ def test_inputs_updated_in_place_before_backward(train_x, twice):
             grads = torch.autograd.grad(sum(v.square().sum() for v in grads), (a, b))
         res.append(grads)
     assert all(torch.equal(p, q) for p, q in zip(*res))
+
+
+def test_no_copies_without_a_graph(monkeypatch):
+    """Evaluation with trainable adapters (no_grad) copies nothing."""
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, _ = _case(sizes, ids, 2, 128, 64, 8)
+    A.requires_grad_(True)
+    want = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B)
+    rets = []
+    orig = nf4_qlora._LoraAdd.apply
+    monkeypatch.setattr(nf4_qlora._LoraAdd, "apply",
+                        lambda *a: rets.append(orig(*a)) or rets[-1])
+    with torch.no_grad():
+        got = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B)
+    assert torch.is_tensor(rets[0]) and torch.equal(got, want.detach())
