@@ -164,7 +164,11 @@ def lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling=1.0):
         eid = expert_ids.to(dev)[nz_d.to(torch.int64)].to(torch.int64)
     else:
         ids = _host_ints(expert_ids)
-        sz_d, eid_d = nf4_grouped.to_device_i32((rows, [ids[g] for g in nz]), dev)
+        ids = [ids[g] for g in nz]
+        E = min(lora_A.shape[0], lora_B.shape[0])
+        if max(ids) >= E:   # (on the device, indexing would abort the process)
+            raise IndexError(f"expert id {max(ids)} is out of range for adapters of {E} experts")
+        sz_d, eid_d = nf4_grouped.to_device_i32((rows, ids), dev)
         eid = eid_d.to(torch.int64)
     sz = sz_d.to(torch.int64)
     # row -> (group, position in group), built on the device; output_size
@@ -214,12 +218,14 @@ def _transforming() -> bool:
             or torch.is_autocast_enabled())
 
 
-def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling) -> bool:
+def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, n_packed) -> bool:
     """Whether the HIP kernels take this low-rank delta: bf16 rows and fp32
     adapters on one GPU, plain contiguous tensors, r % 4 == 0 and r <= 64,
-    widths that are multiples of 8, every row in a group, and a plain number
-    as ``scaling`` (a tensor may be learnable, live on the device or have one
-    value per column: the torch composition multiplies by it)."""
+    widths that are multiples of 8, every row in a group, a plain number as
+    ``scaling`` (a tensor may be learnable, live on the device or have one
+    value per column: the torch composition multiplies by it), and adapters
+    for every expert of the packed stack or for every id known on the host
+    (the kernels add nothing for others; the composition's indexing raises)."""
     if not isinstance(scaling, (int, float)):
         return False
     ts = (out, a_cat, lora_A, lora_B)
@@ -236,7 +242,9 @@ def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling) -> bool:
             and 0 < E <= 65535 and 4 <= r <= 64 and r % 4 == 0 and K % 8 == 0 and N % 8 == 0
             and lora_A.is_contiguous() and lora_B.is_contiguous()
             and lora_A.data_ptr() % 16 == 0 and lora_B.data_ptr() % 16 == 0
-            and T > 0 and sum(int(m) for m in sizes) == T and not _transforming())
+            and T > 0 and sum(int(m) for m in sizes) == T and not _transforming()
+            and (E >= n_packed or not (torch.is_tensor(expert_ids) and expert_ids.is_cuda)
+                 and all(e < E for e, m in zip(_host_ints(expert_ids), sizes) if int(m) > 0)))
 
 
 class _LoraTables:
@@ -372,7 +380,7 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
                                   weights_fn=weights_fn, dgrad_kernel=dgrad_kernel)
     if lora_A is None or lora_B is None:
         return out
-    if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling):
+    if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, packed.shape[0]):
         out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling,
                              torch.is_grad_enabled())
         return out[0] if isinstance(out, tuple) else out

@@ -224,3 +224,23 @@ def test_no_copies_without_a_graph(monkeypatch):
     with torch.no_grad():
         got = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B)
     assert torch.is_tensor(rets[0]) and torch.equal(got, want.detach())
+
+
+def test_adapters_for_fewer_experts_than_the_stack(monkeypatch):
+    """Adapters for the first 2 of 3 experts: ids within them give the delta
+    (an empty group's id does not count), a host id past them raises, and
+    device ids, which nothing on the host can vouch for, take the torch
+    composition and its indexing."""
+    import nf4_qlora
+    sizes, ids = [9, 0, 30], [1, 2, 0]
+    W, S, x, A, B, _ = _case(sizes, ids, 3, 128, 64, 8)
+    want = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, A, B)
+    used = []
+    orig = nf4_qlora._LoraAdd.apply
+    monkeypatch.setattr(nf4_qlora._LoraAdd, "apply", lambda *a: used.append(1) or orig(*a))
+    run = lambda i: nf4_qlora.fused_grouped_lora(x, W, S, sizes, i, A[:2], B[:2])  # noqa: E731
+    assert torch.equal(run(ids), want) and used == [1]
+    with pytest.raises(IndexError):
+        run([1, 0, 2])
+    assert rel_err(run(torch.tensor(ids, device="cuda")), want.double()) <= 1e-3
+    assert used == [1]
