@@ -205,17 +205,21 @@ def _lora_delta_grouped_loop(a_cat, lora_A, lora_B, sizes, expert_ids, scaling=1
 
 # ------------------------------------------------- the fused low-rank kernels --
 
-def _transforming() -> bool:
-    """Whether something other than plain eager autograd watches the torch
-    calls (tracing, functorch transforms, forward-mode, dispatch or function
-    modes, autocast): then the torch composition runs, which they all see."""
-    from torch.autograd import forward_ad
+def _watched() -> bool:
+    """Whether functorch, a dispatch or function mode or a tracer watches the
+    torch calls of this thread."""
     return (torch.compiler.is_compiling() or torch.jit.is_tracing()
             or torch._C._functorch.peek_interpreter_stack() is not None
-            or forward_ad._current_level >= 0
             or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._len_torch_function_stack() > 0
-            or torch.is_autocast_enabled())
+            or torch._C._len_torch_function_stack() > 0)
+
+
+def _transforming() -> bool:
+    """Whether something other than plain eager autograd watches the forward's
+    torch calls (also forward-mode and autocast): then the torch composition
+    runs, which they all see."""
+    from torch.autograd import forward_ad
+    return _watched() or forward_ad._current_level >= 0 or torch.is_autocast_enabled()
 
 
 def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, n_packed) -> bool:
@@ -318,7 +322,8 @@ class _LoraAdd(torch.autograd.Function):
     """``base + bf16(scaling * (a A[e]^T) B[e]^T)`` through the kernels of
     csrc/gnf4_lora.hip (two forward, four backward launches, fp32 sums): the
     values and gradients of adding ``lora_delta_grouped``. A backward that is
-    itself differentiated runs that torch composition instead.
+    itself differentiated, batched (``is_grads_batched``) or watched runs that
+    torch composition instead.
 
     Backward reads copies of the activations and adapters, as the
     composition's gathered ones are: a program may update the adapters, or
@@ -352,12 +357,14 @@ class _LoraAdd(torch.autograd.Function):
             return (g, *(g_copies or (None,) * 3), None, None, None, None)
         a_cat, A, B, u = ctx.saved_tensors
         tb, scaling, need = ctx.tables, ctx.scaling, ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        twice = torch.is_grad_enabled()
+        if (twice or _watched() or type(g) is not torch.Tensor
+                or torch._C._functorch.is_legacy_batchedtensor(g)):
             with torch.enable_grad():
                 ins = [t for t, n in zip((a_cat, A, B), need[1:4]) if n]
                 d = lora_delta_grouped(a_cat, A, B, tb.sizes, tb.expert_ids,
                                        scaling).to(g.dtype)
-                got = iter(torch.autograd.grad(d, ins, g, create_graph=True))
+                got = iter(torch.autograd.grad(d, ins, g, create_graph=twice))
             grads = [next(got) if n else None for n in need[1:4]]
         else:
             s = float(scaling)

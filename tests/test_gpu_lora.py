@@ -244,3 +244,18 @@ def test_adapters_for_fewer_experts_than_the_stack(monkeypatch):
         run([1, 0, 2])
     assert rel_err(run(torch.tensor(ids, device="cuda")), want.double()) <= 1e-3
     assert used == [1]
+
+
+def test_batched_gradients_of_the_adapters():
+    """Several gradients at once (``is_grads_batched``, as vectorised jacobians
+    take them): the rows of one gradient at a time."""
+    import nf4_qlora
+    sizes, ids = [9, 30], [1, 0]
+    W, S, x, A, B, go = _case(sizes, ids, 2, 128, 64, 8)
+    a, b = A.clone().requires_grad_(True), B.clone().requires_grad_(True)
+    out = nf4_qlora.fused_grouped_lora(x, W, S, sizes, ids, a, b, scaling=2.0)
+    gs = torch.stack([go, go * 2, go.flip(0)])
+    got = torch.autograd.grad(out, (a, b), gs, is_grads_batched=True, retain_graph=True)
+    for i, g in enumerate(gs):
+        for p, q in zip(got, torch.autograd.grad(out, (a, b), g, retain_graph=True)):
+            assert rel_err(p[i], q.double()) <= 1e-5
