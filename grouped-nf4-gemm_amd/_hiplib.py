@@ -12,7 +12,7 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "libgnf4_hip.so"
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 FMT_NF4 = 0
 FMT_MXFP4 = 1
@@ -79,6 +79,8 @@ SIGNATURES = {
     "gnf4_hip_lora_up": [_P, _P, _I, _I64, _I64, _I, _P, _P, _P, _I, _I, _F, _P, _I64, _P, _I64,
                          _P],
     "gnf4_hip_lora_wgrad": [_P, _I64, _P, _I, _I64, _I64, _I, _P, _P, _I, _F, _P, _P],
+    "gnf4_hip_lora_wgrad_split": [_P, _I64, _P, _I, _I64, _I64, _I, _P, _P, _P, _I, _I, _F, _P,
+                                  _P, _P],
 }
 
 # entry points that do not return int

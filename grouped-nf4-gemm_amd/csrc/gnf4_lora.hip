@@ -38,13 +38,15 @@ __device__ __forceinline__ float bf16_elem(u32x4_t v, int i) {
 }
 
 struct LoraGroups {
-  const int32_t* tile_off;   // [G + 1] 16-row tiles before a group
+  const int32_t* tile_off;   // [G + 1] tiles before a group
   const int32_t* row_off;    // [G + 1] rows before it
   const int32_t* ids;        // [G] its expert
   int G;
 };
 
-// The tile of workgroup b: one pass over the groups' tile ends, 64 at a time.
+// Tile b of the groups' tiles of kRows rows: one pass over the groups' tile
+// ends, 64 at a time.
+template <int kRows>
 struct LoraTile {
   int row0, rows;
   int64_t e;
@@ -56,9 +58,9 @@ struct LoraTile {
       g += __popcll(__ballot(end <= b));
     }
     g = uniform(g);
-    row0 = t.row_off[g] + 16 * (b - t.tile_off[g]);
+    row0 = t.row_off[g] + kRows * (b - t.tile_off[g]);
     const int left = t.row_off[g + 1] - row0;
-    rows = left < 16 ? left : 16;
+    rows = left < kRows ? left : kRows;
     e = t.ids[g];
   }
 };
@@ -75,7 +77,7 @@ __global__ void __launch_bounds__(256) k_lora_down(const uint16_t* __restrict__ 
   __shared__ f32x4_t red[4][RB][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, q = lane >> 4;
-  const LoraTile t(gr, blockIdx.x);
+  const LoraTile<16> t(gr, blockIdx.x);
   const int row0 = t.row0, rows = t.rows;
   const int64_t e = t.e;
   const bool known = e >= 0 && e < E;
@@ -146,7 +148,7 @@ __global__ void __launch_bounds__(256) k_lora_up(const float* __restrict__ U,
                                                  uint16_t* __restrict__ out, int64_t ldo) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, q = lane >> 4;
-  const LoraTile t(gr, blockIdx.x);
+  const LoraTile<16> t(gr, blockIdx.x);
   const int row0 = t.row0, rows = t.rows;
   const int64_t e = t.e;
   const bool known = e >= 0 && e < E;
@@ -200,9 +202,89 @@ __global__ void __launch_bounds__(256) k_lora_up(const float* __restrict__ U,
   }
 }
 
-// dM[e] = s sum over the expert's rows of P[t, :] Q[t, :]: [C, r] rows, or, kT,
-// [r, C] rows. A wave: one expert, 128 columns of P, all r; MFMA row m of
-// block i is column 8 m + i, contraction over four rows t (lane quarter q).
+// Weight gradients: s sum over rows of P[t, :] Q[t, :], a [C, r] matrix or,
+// kT, [r, C]. A wave: 128 columns of P, all r; MFMA row m of block i is column
+// 8 m + i, contraction over four rows t (lane quarter q).
+template <int RB>
+struct WgradAcc {
+  f32x4_t acc[8][RB];
+  __device__ __forceinline__ WgradAcc() {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int b = 0; b < RB; ++b) acc[i][b] = f32x4_t{};
+  }
+  // adds rows [begin, end); 16 rows' loads at a time
+  __device__ __forceinline__ void add(const uint16_t* __restrict__ P, int64_t ldp,
+                                      const float* __restrict__ Q, int64_t C, int64_t c, int r,
+                                      int begin, int end, int m, int q) {
+    for (int t0 = begin; t0 < end; t0 += 16) {
+      u32x4_t pv[4];
+      float w[4][RB];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + 4 * u + q;
+        const bool in = t < end;
+        pv[u] = in && c < C ? load_a8(P + (int64_t)t * ldp + c) : u32x4_t{};
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          w[u][b] = in && 16 * b + m < r ? Q[(int64_t)t * r + 16 * b + m] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int b = 0; b < RB; ++b)
+            acc[i][b] = mfma4(bf16_elem(pv[u], i), w[u][b], acc[i][b]);
+    }
+  }
+  template <bool kT>
+  __device__ __forceinline__ void store(float* me, int64_t C, int64_t c0, int r, float s, int m,
+                                        int q) const {
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int j = 16 * b + m;
+      if (j >= r) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int64_t n = c0 + 8 * (4 * q + k);
+        if (n >= C) continue;   // C % 8 == 0
+        if constexpr (kT) {
+          f32x4_t v0, v1;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v0[i] = s * acc[i][b][k];
+            v1[i] = s * acc[4 + i][b][k];
+          }
+          f32x4_t* dst = reinterpret_cast<f32x4_t*>(me + (int64_t)j * C + n);
+          dst[0] = v0;
+          dst[1] = v1;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) me[(n + i) * r + j] = s * acc[i][b][k];
+        }
+      }
+    }
+  }
+};
+
+// Calls fn(g) for the groups g of expert e, in order.
+template <class Fn>
+__device__ __forceinline__ void for_groups_of(int e, const int32_t* __restrict__ ids, int G,
+                                              Fn&& fn) {
+  const int lane = threadIdx.x & 63;
+  for (int g0 = 0; g0 < G; g0 += 64) {
+    const int mine = g0 + lane < G ? ids[g0 + lane] : -1;
+    uint64_t hit = __ballot(mine == e);
+    while (hit) {
+      fn(g0 + __ffsll((unsigned long long)hit) - 1);
+      hit &= hit - 1;
+    }
+  }
+}
+
+// One wave per expert and 128 columns: dM[e] over all of the expert's rows.
 // Every expert of the stack is written (zeros where no group has it); groups
 // of one expert are added in group order.
 template <int RB, bool kT>
@@ -216,67 +298,52 @@ __global__ void __launch_bounds__(256) k_lora_wgrad(const uint16_t* __restrict__
   const int e = blockIdx.y;
   const int64_t c0 = ((int64_t)blockIdx.x * 4 + wave) * 128;
   if (c0 >= C) return;
-  const int64_t c = c0 + 8 * m;
-  f32x4_t acc[8][RB];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int b = 0; b < RB; ++b) acc[i][b] = f32x4_t{};
-  for (int g0 = 0; g0 < G; g0 += 64) {
-    const int mine = g0 + lane < G ? ids[g0 + lane] : -1;
-    uint64_t hit = __ballot(mine == e);
-    while (hit) {
-      const int g = g0 + __ffsll((unsigned long long)hit) - 1;
-      hit &= hit - 1;
-      const int end = row_off[g + 1];
-      // 16 rows' loads at a time
-      for (int t0 = row_off[g]; t0 < end; t0 += 16) {
-        u32x4_t pv[4];
-        float w[4][RB];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int t = t0 + 4 * u + q;
-          const bool in = t < end;
-          pv[u] = in && c < C ? load_a8(P + (int64_t)t * ldp + c) : u32x4_t{};
-#pragma unroll
-          for (int b = 0; b < RB; ++b)
-            w[u][b] = in && 16 * b + m < r ? Q[(int64_t)t * r + 16 * b + m] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int b = 0; b < RB; ++b)
-              acc[i][b] = mfma4(bf16_elem(pv[u], i), w[u][b], acc[i][b]);
-      }
-    }
-  }
-  float* me = dM + (int64_t)e * C * r;
-#pragma unroll
-  for (int b = 0; b < RB; ++b) {
-    const int j = 16 * b + m;
-    if (j >= r) continue;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int64_t n = c0 + 8 * (4 * q + k);
-      if (n >= C) continue;   // C % 8 == 0
-      if constexpr (kT) {
-        f32x4_t v0, v1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v0[i] = s * acc[i][b][k];
-          v1[i] = s * acc[4 + i][b][k];
-        }
-        f32x4_t* dst = reinterpret_cast<f32x4_t*>(me + (int64_t)j * C + n);
-        dst[0] = v0;
-        dst[1] = v1;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) me[(n + i) * r + j] = s * acc[i][b][k];
-      }
-    }
-  }
+  WgradAcc<RB> acc;
+  for_groups_of(e, ids, G, [&](int g) {
+    acc.add(P, ldp, Q, C, c0 + 8 * m, r, row_off[g], row_off[g + 1], m, q);
+  });
+  acc.template store<kT>(dM + (int64_t)e * C * r, C, c0, r, s, m, q);
+}
+
+// The same in two launches for experts of many rows: one wave per 256-row
+// chunk of a group and 128 columns writes the chunk's sum to part[chunk], and
+// k_lora_wgrad_sum adds an expert's chunks in order. A wave needs about 1.3
+// (r = 16) to 2.8 us (r = 64) for 16 rows, one after the other, so with a wave
+// per expert the largest expert decides: one of 8192 rows, C = 2048, r = 16 /
+// 64: 650 / 1416 us in k_lora_wgrad, 35 / 66 us here; 8 experts of 512 rows 38
+// / 90 and 24 / 55 us. It is bound by MFMA latency below a round of waves,
+// then by the partial sums' traffic (128 experts of 512 rows: 73 / 228 us in
+// k_lora_wgrad, 79 / 285 us here).
+constexpr int kWgradChunk = 256;
+
+template <int RB, bool kT>
+__global__ void __launch_bounds__(256) k_lora_wgrad_part(const uint16_t* __restrict__ P,
+                                                         int64_t ldp, const float* __restrict__ Q,
+                                                         int64_t C, int r, const LoraGroups gr,
+                                                         float s, float* __restrict__ part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = lane & 15, q = lane >> 4;
+  const int chunk = blockIdx.x;
+  const LoraTile<kWgradChunk> t(gr, chunk);
+  const int64_t c0 = ((int64_t)blockIdx.y * 4 + wave) * 128;
+  if (c0 >= C) return;
+  WgradAcc<RB> acc;
+  acc.add(P, ldp, Q, C, c0 + 8 * m, r, t.row0, t.row0 + t.rows, m, q);
+  acc.template store<kT>(part + (int64_t)chunk * C * r, C, c0, r, s, m, q);
+}
+
+__global__ void __launch_bounds__(256) k_lora_wgrad_sum(const float* __restrict__ part,
+                                                        int64_t n, const LoraGroups gr,
+                                                        float* __restrict__ dM) {
+  const int e = blockIdx.y;
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;   // n % 4 == 0
+  f32x4_t sum{};
+  for_groups_of(e, gr.ids, gr.G, [&](int g) {
+    if (i < n)
+      for (int64_t k = gr.tile_off[g]; k < gr.tile_off[g + 1]; ++k)
+        sum += *reinterpret_cast<const f32x4_t*>(part + k * n + i);
+  });
+  if (i < n) *reinterpret_cast<f32x4_t*>(dM + (int64_t)e * n + i) = sum;
 }
 
 template <class Fn>
@@ -366,6 +433,34 @@ int gnf4_hip_lora_wgrad(const void* p, int64_t ldp, const float* q, int transpos
     else
       hipLaunchKernelGGL((k_lora_wgrad<rb, false>), grid, dim3(256), 0, s,
                          static_cast<const uint16_t*>(p), ldp, q, C, r, expert_ids, row_off, G, scale, dw);
+  });
+}
+
+int gnf4_hip_lora_wgrad_split(const void* p, int64_t ldp, const float* q, int transposed,
+                              int64_t E, int64_t C, int r, const int32_t* chunk_off,
+                              const int32_t* row_off, const int32_t* expert_ids, int G,
+                              int n_chunks, float scale, float* part, float* dw, void* stream) {
+  if (G <= 0 || n_chunks <= 0 || E <= 0 || E > 65535 || C <= 0 || C % 8 || !rank_ok(r) ||
+      ldp < C || ldp % 8)
+    return -1;
+  if (!p || !q || !chunk_off || !row_off || !expert_ids || !part || !dw || !al16(p) ||
+      !al16(part) || !al16(dw))
+    return -1;
+  const int64_t gy = (C + 511) / 512, n = C * r, gx = (n / 4 + 255) / 256;
+  if (gy > 65535 || gx > 0x7FFFFFFF) return -1;
+  const LoraGroups gr{chunk_off, row_off, expert_ids, G};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)n_chunks, (unsigned)gy);
+  return by_rank(r, [&](auto RB) {
+    constexpr int rb = decltype(RB)::value;
+    if (transposed)
+      hipLaunchKernelGGL((k_lora_wgrad_part<rb, true>), grid, dim3(256), 0, s,
+                         static_cast<const uint16_t*>(p), ldp, q, C, r, gr, scale, part);
+    else
+      hipLaunchKernelGGL((k_lora_wgrad_part<rb, false>), grid, dim3(256), 0, s,
+                         static_cast<const uint16_t*>(p), ldp, q, C, r, gr, scale, part);
+    hipLaunchKernelGGL(k_lora_wgrad_sum, dim3((unsigned)gx, (unsigned)E), dim3(256), 0, s, part,
+                       n, gr, dw);
   });
 }
 

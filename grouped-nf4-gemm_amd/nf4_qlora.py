@@ -251,6 +251,10 @@ def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, n_pack
                  and all(e < E for e, m in zip(_host_ints(expert_ids), sizes) if int(m) > 0)))
 
 
+# Rows of a chunk of gnf4_hip_lora_wgrad_split
+_WGRAD_CHUNK = 256
+
+
 class _LoraTables:
     """Device tables of one routing: tile and row offsets, expert ids. Nothing
     of the caller's is kept: it may write the next layer's routing into the
@@ -259,17 +263,33 @@ class _LoraTables:
     def __init__(self, sizes, expert_ids, dev):
         self.sizes = [int(v) for v in sizes]
         m = np.asarray(self.sizes, dtype=np.int32)
-        off = np.zeros((2, len(m) + 1), dtype=np.int32)
+        off = np.zeros((3, len(m) + 1), dtype=np.int32)
         np.cumsum((m + 15) // 16, out=off[0, 1:])
         np.cumsum(m, out=off[1, 1:])
+        np.cumsum((m + _WGRAD_CHUNK - 1) // _WGRAD_CHUNK, out=off[2, 1:])
         on_dev = torch.is_tensor(expert_ids) and expert_ids.is_cuda
         ids = [] if on_dev else [nf4_grouped._np_ids(expert_ids)]
         views = nf4_grouped.to_device_i32([*off, *ids], dev)
         self.n, self.G = int(off[0, -1]), len(m)
-        self.tile_off, self.row_off = views[:2]
+        self.n_chunks = int(off[2, -1])
+        self.tile_off, self.row_off, self.chunk_off = views[:3]
         self.ids = (torch.empty(self.G, dtype=torch.int32, device=dev).copy_(expert_ids)
-                    if on_dev else views[2])
+                    if on_dev else views[3])
         self.expert_ids = self.ids if on_dev else ids[0].tolist()   # for the composition
+        # the most rows an expert has (device ids: of one group)
+        self.most = int(m.max() if on_dev else np.bincount(ids[0], m).max())
+
+    def split_rows(self, E) -> bool:
+        """Whether the adapter gradients take the kernel that splits an
+        expert's rows over waves: where one wave per expert would run long
+        (from 384 rows) while other waves idle (fewer than 32 such experts'
+        worth of rows). Direct and split, MI355X, K = 2048, r = 16, even
+        groups: 8 experts of 320 / 384 / 512 / 4096 rows 25 / 29 / 38 / 328
+        and 23 / 23 / 24 / 46 us; 32 experts of 320 / 384 / 1024 31 / 36 / 88
+        and 31 / 32 / 44 us; 64 experts of 384 / 512 / 1024 39 / 50 / 101 and
+        45 / 45 / 75 us, at r = 64 90 / 113 / 211 and 132 / 133 / 275 us. More
+        device ids than experts: some are repeated, so it splits."""
+        return self.most >= 384 and 32 * self.most >= sum(self.sizes) or self.G > E
 
     def args(self):
         return (self.tile_off.data_ptr(), self.row_off.data_ptr(), self.ids.data_ptr(), self.G,
@@ -312,9 +332,16 @@ def _lora_up(u, w, transposed, C, tb, scale, base=None):
 
 def _lora_wgrad(p, q, like, transposed, tb, scale):
     dw = torch.empty_like(like)
+    E, C, r = like.shape[0], p.shape[1], q.shape[1]
+    if tb.split_rows(E):
+        part = torch.empty(tb.n_chunks, C * r, dtype=torch.float32, device=p.device)
+        _lora_call("gnf4_hip_lora_wgrad_split", p.device, p.data_ptr(), p.stride(0), q.data_ptr(),
+                   transposed, E, C, r, tb.chunk_off.data_ptr(), tb.row_off.data_ptr(),
+                   tb.ids.data_ptr(), tb.G, tb.n_chunks, scale, part.data_ptr(), dw.data_ptr())
+        return dw
     _lora_call("gnf4_hip_lora_wgrad", p.device, p.data_ptr(), p.stride(0), q.data_ptr(),
-               transposed, like.shape[0], p.shape[1], q.shape[1], tb.ids.data_ptr(),
-               tb.row_off.data_ptr(), tb.G, scale, dw.data_ptr())
+               transposed, E, C, r, tb.ids.data_ptr(), tb.row_off.data_ptr(), tb.G, scale,
+               dw.data_ptr())
     return dw
 
 

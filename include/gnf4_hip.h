@@ -53,7 +53,7 @@
 extern "C" {
 #endif
 
-#define GNF4_HIP_ABI_VERSION 15
+#define GNF4_HIP_ABI_VERSION 16
 
 #define GNF4_FMT_NF4 0
 #define GNF4_FMT_MXFP4 1
@@ -480,6 +480,16 @@ int gnf4_hip_lora_up(const float *u, const float *w, int transposed, int64_t E, 
 int gnf4_hip_lora_wgrad(const void *p, int64_t ldp, const float *q, int transposed, int64_t E,
                         int64_t C, int r, const int32_t *expert_ids, const int32_t *row_off,
                         int G, float scale, float *dw, void *stream);
+
+/* gnf4_hip_lora_wgrad for experts of many rows, which it takes one after the
+ * other: group g's rows are cut into chunks chunk_off[g] .. chunk_off[g + 1]
+ * ([G + 1]) of at most 256 rows, n_chunks = chunk_off[G]; part is scratch of
+ * n_chunks * C * r floats, 16-byte aligned. An expert's chunks are added in
+ * order (not the bits of gnf4_hip_lora_wgrad). */
+int gnf4_hip_lora_wgrad_split(const void *p, int64_t ldp, const float *q, int transposed,
+                              int64_t E, int64_t C, int r, const int32_t *chunk_off,
+                              const int32_t *row_off, const int32_t *expert_ids, int G,
+                              int n_chunks, float scale, float *part, float *dw, void *stream);
 
 #ifdef __cplusplus
 }

@@ -259,3 +259,39 @@ def test_batched_gradients_of_the_adapters():
     for i, g in enumerate(gs):
         for p, q in zip(got, torch.autograd.grad(out, (a, b), g, retain_graph=True)):
             assert rel_err(p[i], q.double()) <= 1e-5
+
+
+@pytest.mark.parametrize("sizes,ids,E,K,N,r,split", [
+    ([383, 64], [1, 0], 3, 128, 64, 16, False),           # the rule's line
+    ([384, 64], [1, 0], 3, 128, 64, 16, True),
+    ([384] * 33, list(range(33)), 33, 64, 64, 4, False),  # enough experts to fill the waves
+    ([200, 0, 200, 7], [2, 0, 2, 1], 3, 576, 1032, 20, True),   # one expert in two groups
+    ([255, 256, 257, 513], [3, 0, 2, 1], 70, 2048, 72, 64, True),
+    ([1] * 70 + [769], list(range(71)), 72, 64, 520, 32, True),   # groups past a lane pass
+])
+@pytest.mark.parametrize("dev_ids", [False, True])
+def test_adapter_gradients_of_long_groups(sizes, ids, E, K, N, r, split, dev_ids, monkeypatch):
+    """The kernel that splits an expert's rows into 256-row chunks, at the
+    chunks' edges and on both sides of the rule that takes it (device ids: by
+    the largest group), against float64 (fp32 sums of at most 1000 terms,
+    inputs and the two-step products rounded to fp32: 1e-5)."""
+    import nf4_qlora
+    W, S, x, A, B, go = _case(sizes, ids, E, K, N, r)
+    arg = torch.tensor(ids, device="cuda") if dev_ids else ids
+    if dev_ids and max(sizes) < 384:
+        split = len(ids) > E
+    names = []
+    orig = nf4_qlora._lora_call
+    monkeypatch.setattr(nf4_qlora, "_lora_call", lambda n, *a: names.append(n) or orig(n, *a))
+    _out, _gx, gA, gB = _run(True, W, S, x, A, B, go, sizes, arg, monkeypatch)
+    assert names.count("gnf4_hip_lora_wgrad_split") == (2 if split else 0)
+    assert names.count("gnf4_hip_lora_wgrad") == (0 if split else 2)
+    wA, wB, row = torch.zeros_like(A).double(), torch.zeros_like(B).double(), 0
+    for m, e in zip(sizes, ids):
+        xe, g = x[row:row + m].double(), go[row:row + m].double()
+        wA[e] += 2 * (g @ B[e].double()).t() @ xe
+        wB[e] += 2 * g.t() @ (xe @ A[e].double().t())
+        row += m
+    assert rel_err(gA, wA) <= 1e-5 and rel_err(gB, wB) <= 1e-5
+    unused = [e for e in range(E) if e not in ids]
+    assert not gA[unused].any() and not gB[unused].any()
