@@ -3591,20 +3591,24 @@ int launch_fwd(const FwdArgs& p, int block_m, hipStream_t stream, const PwTiles*
     if (rc) return rc;
   } else {
     // k_tile_fwd: tables of any height up to 256 rows (each row is computed
-    // the same way in every tile), whole 64-wide k steps, 4-column stores
-    const bool tile_ok = p.N % 4 == 0 && p.ldo % 4 == 0 && p.K % kPfBK == 0 &&
-                         (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM &&
-                         (int64_t)kPtBM * p.lda * 2 < 0x7FFFFFFF &&
-                         (int64_t)kPtBM * p.ldo * 2 < 0x7FFFFFFF;
-    if (tile_ok) {
+    // the same way in every tile), whole 64-wide k steps, 4-column stores, and
+    // a tile's rows within 32-bit offsets
+    const bool shape_ok = p.N % 4 == 0 && p.ldo % 4 == 0 && p.K % kPfBK == 0 &&
+                          (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM;
+    const bool fits = (int64_t)kPtBM * p.lda * 2 < 0x7FFFFFFF &&
+                      (int64_t)kPtBM * p.ldo * 2 < 0x7FFFFFFF && kPfBN * p.sbn < 0x7FFFFFFF &&
+                      kPfBN * p.ssn * 4 < 0x7FFFFFFF;
+    if (shape_ok && fits) {
       const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kPfBN - 1) / kPfBN);
       // the grid covers eight equal XCD ranges
       const int64_t per_x = tiles_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
       return launch_tile_fwd(FMT, p, tt ? *tt : no_tiles(), per_x, stream);
     }
-    // kernel-argument tables and 256-row tables are for that kernel only
-    if (tt || block_m > kPfBM) return -1;
+    // kernel-argument tables and 256-row tables are for that kernel only; the
+    // caller may upload a table of lower tiles instead
+    if (tt) return shape_ok ? 1 : -1;
+    if (block_m > kPfBM) return -1;
     const int64_t tiles = (int64_t)p.n_mtiles * ((p.N + kBN - 1) / kBN);
     const int64_t grid = clamp_grid(tiles, cus);
     switch (block_m) {
@@ -3626,12 +3630,13 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
   {
     // the tiles with transposed tr8 reads of the packed rows: at most 256
     // rows, whole 64-wide n steps and 64-wide k blocks
-    const bool w_ok = p.N % kDgStep == 0 && p.K % 64 == 0 && p.ldo % 4 == 0 &&
-                      (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM &&
-                      (int64_t)kPtBM * p.ldg * 2 < 0x7FFFFFFF &&
+    const bool shape_ok = p.N % kDgStep == 0 && p.K % 64 == 0 && p.ldo % 4 == 0 &&
+                          (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPtBM;
+    const bool fits = (int64_t)kPtBM * p.ldg * 2 < 0x7FFFFFFF &&
                       (int64_t)kPtBM * p.ldo * 2 < 0x7FFFFFFF && p.N * p.sbn < 0x7FFFFFFF &&
                       p.N * p.ssn * 4 < 0x7FFFFFFF;
-    if (w_ok) {
+    if (tt && !(shape_ok && fits)) return shape_ok ? 1 : -1;
+    if (shape_ok && fits) {
       FwdArgs f{};
       f.a = p.g;
       f.lda = p.ldg;
@@ -3669,9 +3674,6 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
       return hipGetLastError() == hipSuccess ? 0 : -2;
     }
   }
-  // a kernel-argument tile table is for those two only: the others read
-  // device tables
-  if (tt) return -1;
   const bool tiled_ok = p.N % kDgStep == 0 && p.ldo % 4 == 0 &&
                         (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 && block_m <= kPfBM &&
                         (int64_t)kPfBM * p.ldg * 2 < 0x7FFFFFFF && p.N * p.sbn < 0x7FFFFFFF;

@@ -557,18 +557,22 @@ def _tall_tiles_ok(N: int, K: int) -> bool:
 def _fwd_block_m(max_m: int, N: int, K: int, block_m=None) -> int:
     """Tile height of a tiled forward launch, shared by the op and by
     ``GroupPlan``: the caller's ``block_m`` rounded up to a supported height,
-    else 256 rows wherever the shape takes them (a tile computes only its
-    group's 32-row subtiles, and each decoded weight feeds all of them), else
-    the reference's group-size rule. Against 128-row tiles with every subtile
-    computed (MI355X): 128 experts, N = 2048, K = 768, 32 / 64 / 128 rows per
-    group 47.9 / 56.0 / 72.0 us against 61.0 / 68.5 / 88.1; 64 experts, N =
-    2048, K = 256, 32 / 128 rows 15.4 / 21.8 against 18.6 / 29.8; MXFP4, K =
-    512, 14.8 / 26.3 against 23.2 / 36.6."""
+    else 256 rows for groups above 128 wherever the shape takes them, else the
+    reference's group-size rule: one tile per group, which the tile kernel
+    (it computes only a tile's 32-row subtiles) and, for strides and outputs
+    it does not take, the general one both run."""
     if block_m is not None:
         return _kernel_block_m(block_m)
-    if _tall_tiles_ok(N, K):
+    if max_m > 128 and _tall_tiles_ok(N, K):
         return 256
     return _kernel_block_m(_prefill_block_m(max_m))
+
+
+def _tile_kernel_order(bm: int, N: int, K: int, block_m) -> bool:
+    """Whether a tiled forward launch orders its tiles for the persistent tile
+    kernel and passes them in its arguments: 256-row tables and every table of
+    a shape it takes, except those of a caller's own lower height."""
+    return bm == 256 or block_m is None and _tall_tiles_ok(N, K)
 
 
 # ------------------------------------------------------------------ launch --
@@ -711,13 +715,14 @@ class GroupPlan:
         """(block_m, (t_row0, t_rows, t_group) on the device) for a weight
         shape: the tile height the op would use."""
         bm = _fwd_block_m(self.max_m, N, K, self.user_block_m)
-        if bm not in self._tables:
+        key = bm, _tile_kernel_order(bm, N, K, self.user_block_m)
+        if key not in self._tables:
             t0, tr, tg = _tiles_host(self.sizes, bm)
-            if bm == 256:
+            if key[1]:
                 t0, tr, tg = _xcd_balanced(t0, tr, tg)
-            self._tables[bm] = tuple(torch.tensor(v, dtype=torch.int32, device=self.device)
-                                     for v in (t0, tr, tg))
-        return bm, self._tables[bm]
+            self._tables[key] = tuple(torch.tensor(v, dtype=torch.int32, device=self.device)
+                                      for v in (t0, tr, tg))
+        return bm, self._tables[key]
 
     def args(self, N: int, K: int):
         if self.decode:
@@ -853,7 +858,7 @@ def _launch_fwd(fmt: int, a_cat, W, S, sizes, expert_ids, block_m, op, fp32w=Fal
     else:
         bm = _fwd_block_m(max_m, N, K, block_m)
         t0, tr, tg = _tiles_np(sizes_i, bm)
-        if bm == 256:
+        if _tile_kernel_order(bm, N, K, block_m):
             t0, tr, tg = _xcd_balanced(t0, tr, tg)
             if len(t0) <= ARG_TILES_MAX:
                 a0, ar, ag, is_e, e_ptr = _arg_tiles(t0, tr, tg, eids_dev, expert_ids)

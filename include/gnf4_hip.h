@@ -38,7 +38,8 @@
  *                    of 0 rows may stand anywhere: nothing to do). With
  *                    K % 64 == 0, N % 4 == 0, ldo % 4 == 0 and an 8-byte
  *                    aligned out every height runs the eight-wave tile
- *                    kernel; 256 needs them (-1 otherwise). The order is free
+ *                    kernel (unless 256 rows of an operand span 2 GiB or
+ *                    more); 256 needs it (-1 otherwise). The order is free
  *                    (each XCD takes a contiguous eighth of the list).
  *
  * Return codes (the reference CPU tier's convention, gnf4_native/cpu_kernels.c:745-761):
@@ -175,8 +176,10 @@ int gnf4_hip_grouped_decode_routed(int fmt, const void *a, int a_dtype, int64_t 
  * host arrays of n_mtiles int32, read before the call returns. With
  * tile_group_is_expert = 1, tile_group holds each tile's expert id and
  * expert_ids may be NULL; otherwise it holds group indices into the device
- * array expert_ids. Returns 1, launching nothing, when n_mtiles > 256 (the
- * caller uploads the table and calls gnf4_hip_grouped_fwd), -1 on a shape
+ * array expert_ids. Returns 1, launching nothing, when n_mtiles > 256 or the
+ * strides exceed the kernel's 32-bit offsets (256 rows of a, out, B or the
+ * scales span 2 GiB or more): the caller uploads the table, of tiles of at
+ * most 128 rows for such strides, and calls gnf4_hip_grouped_fwd. -1 on a shape
  * the 256-row kernel does not take or an inconsistent table. Replaces the
  * same launch as gnf4_hip_grouped_fwd, reference
  * kernel/nf4_grouped.py:750-906 (its tile tables go through
@@ -361,7 +364,9 @@ int gnf4_hip_grouped_dgrad(int fmt, const void *grad_out, int g_dtype, int64_t l
  * kernel's arguments (as gnf4_hip_grouped_fwd_tiles): same bits as
  * gnf4_hip_grouped_dgrad with the same table. Needs N % 64 == 0 and
  * K % 64 == 0 (-1 otherwise); returns 1 without launching when
- * n_mtiles > 256. Replaces the launch of dgrad_4bit_grouped, reference
+ * n_mtiles > 256 or the strides exceed its 32-bit offsets (256 rows of
+ * grad_out or out, or an expert's packed rows or scales, span 2 GiB or more;
+ * gnf4_hip_grouped_dgrad takes these at block_m <= 128). Replaces the launch of dgrad_4bit_grouped, reference
  * kernel/nf4_grouped.py:1100-1120. */
 int gnf4_hip_grouped_dgrad_tiles(int fmt, const void *grad_out, int g_dtype, int64_t ldg,
                                  const uint8_t *B, int64_t stride_be, int64_t stride_bn,

@@ -111,3 +111,59 @@ def test_empty_tiles_in_a_device_table(fmt, kind, bm, K, empty):
     ref = torch.cat([x[r0:r0 + m].double() @ (w[i % 4].t() if kind == "fwd" else w[i % 4])
                      for i, (r0, m) in enumerate(zip(row0.tolist(), rows.tolist())) if m])
     assert rel_err(got, ref) <= 1e-2
+
+
+def _spread(t, stride):
+    """``t [T, C]`` in rows ``stride`` elements apart."""
+    T, C = t.shape
+    buf = torch.empty((T - 1) * stride + C, dtype=t.dtype, device="cuda")
+    return buf.as_strided((T, C), (stride, 1)).copy_(t)
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
+@pytest.mark.parametrize("kind", ["fwd", "dgrad"])
+@pytest.mark.parametrize("which", ["rows", "weights"])
+def test_strides_past_the_tile_kernels_offsets(fmt, kind, which):
+    """Rows so far apart that 256 of them (of an expert's packed rows, in the
+    dgrad) span 2 GiB: the tile kernels' 32-bit offsets do not reach them and
+    the general kernels run. Host and device ids."""
+    from test_gpu_dgrad import _ops as dgrad_ops
+    N, K, sizes, ids = 64, 128, [20, 3, 17], [0, 1, 0]
+    W, S = _stack(fmt, 2, N, K, seed=3)
+    x = rand_acts(sum(sizes), K if kind == "fwd" else N, seed=4)
+    op = (_ops() if kind == "fwd" else dgrad_ops())[fmt]
+    want = op(x, W, S, sizes, ids)
+    xs, Ws = x, W
+    if which == "rows":
+        xs = _spread(x, 1 << 22)
+    else:
+        # one row of both experts in turn, 2^31 / 256 (forward) or / 64 apart
+        step = 1 << (23 if kind == "fwd" else 25)
+        buf = torch.empty((N - 1) * step + 2 * K, dtype=torch.uint8, device="cuda")
+        Ws = buf.as_strided(W.shape, (K, step, 1)).copy_(W)
+    for arg in (ids, torch.tensor(ids, device="cuda")):
+        got = op(xs, Ws, S, sizes, arg)
+        assert rel_err(got, want.double()) <= 1e-3   # another order of fp32 sums
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("K", [256, 1024])
+def test_planned_launch_into_an_output_off_the_tile_kernels_alignment(fmt, K):
+    """A plan's launch may write into columns of a wider buffer: an odd row
+    stride or offset, which the tile kernel's 8-byte stores do not take, runs
+    the general kernel, with and without tables built for the shape."""
+    import nf4_grouped
+    name, N, sizes, ids = ("nf4", "mxfp4")[fmt], 72, [40, 128, 5], [2, 0, 1]
+    W, S = _stack(name, 3, N, K, seed=5)
+    a = rand_acts(sum(sizes), K, seed=6)
+    want = _ops()[name](a, W, S, sizes, ids)
+    for shape in (None, (N, K)):
+        plan = nf4_grouped.GroupPlan(sizes, ids, "cuda", shape=shape)
+        for off, width in ((1, N + 3), (2, N + 4), (0, N + 2)):
+            buf = torch.full((sum(sizes), width), 7.0, dtype=torch.bfloat16, device="cuda")
+            out = buf[:, off:off + N]
+            nf4_grouped.launch_planned(fmt, a, W, S, plan, out=out)
+            assert rel_err(out, want.double()) <= 1e-3
+            out.fill_(7)
+            assert bool((buf == 7).all())
+        assert torch.equal(nf4_grouped.launch_planned(fmt, a, W, S, plan), want)
