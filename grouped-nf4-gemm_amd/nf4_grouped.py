@@ -439,23 +439,31 @@ def _tiles_np(sizes_i, block_m: int):
 
 
 def _xcd_balanced(t_row0, t_rows, t_group):
-    """Order tiles for the persistent kernels, which hand XCD x the x-th contiguous eighth of the tile list: the tiles, largest height class
-    first (group order within a class), are dealt round robin to 8 bins,
-    which then run back to back. Each bin gets an equal share of every
-    class and runs its largest tiles first. Only the order changes; every
-    output row is computed the same way. O(n), no sort: the input is in group
-    order already."""
+    """Order tiles for the persistent kernels, which hand XCD x the x-th
+    contiguous eighth of the tile list: the tiles, largest height class first
+    (group order within a class), are dealt round robin to 8 bins, which then
+    run back to back. Each bin gets an equal share of every class and runs its
+    largest tiles first; of a single class every eighth is an equal share as
+    it is. Only the order changes; every output row is computed the same way."""
     n = len(t_row0)
     if n < 16:
         return t_row0, t_rows, t_group
     if isinstance(t_rows, np.ndarray):
-        cls = (t_rows > 128).astype(np.int8) * 2 + ((t_rows > 64) & (t_rows <= 128))
-        ranked = np.concatenate([np.nonzero(cls == c)[0] for c in (2, 1, 0)])
-        order = np.concatenate([ranked[x::8] for x in range(8)])
+        over64, over128 = t_rows > 64, t_rows > 128
+        n64, n128 = np.count_nonzero(over64), np.count_nonzero(over128)
+        if n64 == 0 or n128 == n or (n64 == n and n128 == 0):
+            return t_row0, t_rows, t_group
+        order = np.full(-(-n // 8) * 8, -1)
+        order[:n] = np.argsort(-(over64.view(np.int8) + over128.view(np.int8)), kind="stable")
+        order = order.reshape(-1, 8).T.ravel()
+        if n % 8:
+            order = order[order >= 0]
         return t_row0[order], t_rows[order], t_group[order]
     by_class = ([], [], [])
     for i, r in enumerate(t_rows):
         by_class[2 if r > 128 else (1 if r > 64 else 0)].append(i)
+    if max(map(len, by_class)) == n:
+        return t_row0, t_rows, t_group
     ranked = by_class[2] + by_class[1] + by_class[0]
     order = [i for x in range(8) for i in ranked[x::8]]
     return ([t_row0[i] for i in order], [t_rows[i] for i in order],
