@@ -391,6 +391,16 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14));
 }
 
+// Between LDS writes and reads of one wave that hand data from lane to lane
+// without a workgroup barrier. The LDS serves a wave's accesses in order, so
+// nothing waits; but to the compiler each lane is a thread of its own, and it
+// may keep the value of an earlier read on the path of the lanes that did not
+// write since.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // Values the kernel knows to be wave-uniform but the compiler may not (it

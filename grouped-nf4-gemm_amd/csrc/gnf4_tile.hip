@@ -1031,6 +1031,7 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
         for (int g = 0; g < 4; ++g)
           *reinterpret_cast<u32x4_t*>(ob + (l32 & 15) * 128 + (((2 * g + h) ^ (l32 & 7)) << 4)) =
               v[g];
+      wave_lds_fence();
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int row = j * 8 + (lane >> 3);
@@ -1038,6 +1039,7 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
             *reinterpret_cast<const u32x4_t*>(ob + row * 128 + (((lane & 7) ^ (row & 7)) << 4));
         store_b128(o, ro, coff, uniform((i * 32 + r16 * 16 + j * 8) * ldo2));
       }
+      wave_lds_fence();
     }
   }
   if (F == 1) {
