@@ -373,15 +373,12 @@ __device__ __forceinline__ float load_scale(const FwdArgs& p, int64_t e, int64_t
 // cache-policy operand of a buffer store: nt (non-temporal) on gfx950
 constexpr int kNonTemporal = 2;
 
-// A 16-byte non-temporal buffer store at a scalar offset. The store reads its
-// data registers after it issues: a VALU write to one of them in the very next
-// instruction (which the compiler allows at a scalar offset) replaced that
-// dword of the stored data, so idle cycles follow the store.
-__device__ __forceinline__ void store_b128(u32x4_t v, __amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, kNonTemporal);
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 1");
-  __builtin_amdgcn_sched_barrier(0);
+// A 16-byte non-temporal buffer store. The offset is the lane's alone: the
+// store reads its data registers after it issues, and behind a store with a
+// scalar offset as well the compiler allows a VALU write to one of them in the
+// very next instruction, which replaced that dword of the stored data.
+__device__ __forceinline__ void store_b128(u32x4_t v, __amdgpu_buffer_rsrc_t r, int voff) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, 0, kNonTemporal);
 }
 
 // s_waitcnt with vmcnt(n) and lgkmcnt(0), expcnt untouched (gfx9 encoding).

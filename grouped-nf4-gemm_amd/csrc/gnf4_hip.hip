@@ -2400,13 +2400,12 @@ __device__ __forceinline__ void dgrad_tall_tile(const FwdArgs& p, const PfTile t
   const int chunk = lane & 31;
   const int col = t.n0 + chunk * 8;
   const int coff = col < p.K ? col * 2 + h * ldo2 : kOOB;   // K % 64 == 0
-  // wave w stores rows 2 (4 j + w) + lane / 32, j = 0 .. 4 kM - 1 (no scalar
-  // offset: see store_b128)
+  // wave w stores rows 2 (4 j + w) + lane / 32, j = 0 .. 4 kM - 1
 #pragma unroll
   for (int j = 0; j < kM * 4; ++j) {
     const int row = (j * 4 + wave) * 2 + h;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(smem + row * 512 + ((chunk ^ (row & 31)) << 4));
-    __builtin_amdgcn_raw_buffer_store_b128(v, ro, coff + (j * 4 + wave) * 2 * ldo2, 0, kNonTemporal);
+    store_b128(v, ro, coff + (j * 4 + wave) * 2 * ldo2);
   }
 }
 

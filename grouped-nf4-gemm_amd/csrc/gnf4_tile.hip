@@ -580,7 +580,7 @@ __device__ __forceinline__ int tile_fwd(const FwdArgs& p, const PfTile t, const 
       const u32x4_t v =
           *reinterpret_cast<const u32x4_t*>(ob + row * 512 + ((r32 ^ (row & 31)) << 4));
       const int so = uniform((r0 * 32 + (j * 8 + wave) * 2) * ldo2);
-      store_b128(v, ro, coff16, so);
+      store_b128(v, ro, coff16 + so);
       if (straddle) {
         u32x2_t v2;
         v2.x = v[0];
@@ -1037,7 +1037,7 @@ __device__ __forceinline__ DgradPos tile_dgrad(const FwdArgs& p, const PfTile t,
         const int row = j * 8 + (lane >> 3);
         const u32x4_t o =
             *reinterpret_cast<const u32x4_t*>(ob + row * 128 + (((lane & 7) ^ (row & 7)) << 4));
-        store_b128(o, ro, coff, uniform((i * 32 + r16 * 16 + j * 8) * ldo2));
+        store_b128(o, ro, coff + (i * 32 + r16 * 16 + j * 8) * ldo2);
       }
       wave_lds_fence();
     }
