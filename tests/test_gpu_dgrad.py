@@ -193,12 +193,27 @@ def test_dgrad_tall_several_tiles_per_workgroup(fmt):
         assert torch.equal(got[g * T:(g + 1) * T], dec[rows % N]), g
 
 
+def _runs_wide_tiles(n_mtiles, K, rows):
+    """Whether the library runs 512-column tiles for a table of tiles of at
+    most ``rows`` rows: at most 160, and at most 5/9 of the rounds over the
+    compute units that 256-column tiles need."""
+    import _hiplib
+    cus = _hiplib.load().gnf4_hip_device_cus()
+    rounds = lambda cols: -(-n_mtiles * -(-K // cols) // cus)  # noqa: E731
+    return rows <= 160 and 9 * rounds(512) <= 5 * rounds(256)
+
+
 @pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
 @pytest.mark.parametrize("G,N,K,rows,pads", [
     (150, 64, 320, (1, 31, 32, 33), (0, 0, 0, 0)),        # one step, half a 512-column tile
-    (150, 128, 576, (64, 65, 96, 128), (8, 4, 1, 4)),     # two steps, a 64-column tail tile
+    (128, 128, 576, (64, 65, 96, 128), (8, 4, 1, 4)),     # two steps, a 64-column tail tile
     (150, 192, 512, (127, 97, 2, 128), (16, 20, 3, 8)),
-    (300, 320, 1024, (128, 5, 63, 34), (0, 16, 2, 64)),   # several tiles per workgroup
+    # several tiles per workgroup, after 1, 2, 3 and 5 steps
+    (512, 64, 512, (33, 1, 128, 70), (0, 0, 0, 0)),
+    (512, 128, 512, (128, 32, 5, 96), (8, 4, 1, 4)),
+    (256, 192, 1024, (64, 128, 17, 100), (0, 0, 0, 8)),
+    (256, 320, 1024, (128, 5, 63, 34), (0, 16, 2, 64)),
+    (640, 128, 960, (20, 90, 128, 40), (0, 0, 0, 0)),     # five, with tail columns
 ])
 def test_dgrad_wide_tiles_give_the_tall_kernels_bits(fmt, G, N, K, rows, pads):
     """Tables of at most 128 rows over enough groups run 512-column tiles;
@@ -207,6 +222,7 @@ def test_dgrad_wide_tiles_give_the_tall_kernels_bits(fmt, G, N, K, rows, pads):
     groups on both sides of each 32-row subtile. Against fp64: one bf16
     rounding of the weights and one of the result (2^-8 each, relative to the
     sum of magnitudes) and N fp32 additions."""
+    assert _runs_wide_tiles(G, K, 128) and not _runs_wide_tiles(G, K, 256)
     import _hiplib
     W, S = _stack(fmt, 8, N, K, seed=21)
     sizes = [rows[g % 4] for g in range(G)]
@@ -248,14 +264,17 @@ def test_dgrad_wide_tiles_give_the_tall_kernels_bits(fmt, G, N, K, rows, pads):
 
 @pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
 @pytest.mark.parametrize("rows", [(129, 160, 1, 145), (130, 161, 96, 33)])
-@pytest.mark.parametrize("N", [64, 128, 320])
-def test_dgrad_wide_tiles_up_to_160_rows(fmt, rows, N, monkeypatch):
+@pytest.mark.parametrize("N,G,K", [(64, 128, 576), (128, 128, 576), (320, 128, 576),
+                                   (64, 256, 1024), (128, 256, 1024), (192, 256, 1024)])
+def test_dgrad_wide_tiles_up_to_160_rows(fmt, rows, N, G, K, monkeypatch):
     """A table in the kernel's arguments shows its largest tile: up to 160 rows
-    run 512-column tiles (161 do not). The uploaded 256-row table runs the
-    256-row kernel: the same bits, and fp64 within one bf16 rounding of the
-    weights, one of the result and N fp32 additions."""
+    run 512-column tiles (161 do not), one per workgroup or several. The
+    uploaded 256-row table runs the 256-row kernel: the same bits, and fp64
+    within one bf16 rounding of the weights, one of the result and N fp32
+    additions."""
     import nf4_grouped
-    G, K = 150, 576
+    assert _runs_wide_tiles(G, K, max(rows)) == (max(rows) <= 160)
+    assert G <= nf4_grouped.ARG_TILES_MAX
     W, S = _stack(fmt, 8, N, K, seed=31)
     sizes = [rows[g % 4] for g in range(G)]
     ids = [(5 * g) % 8 for g in range(G)]
