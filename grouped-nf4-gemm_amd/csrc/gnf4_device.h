@@ -125,22 +125,6 @@ __device__ __forceinline__ u32x4_t nf4_dword_to_bf16(const float2* tab, unsigned
   return r;
 }
 
-// Same, with the table at an LDS address below 16 MiB whose bits 8..15 are
-// zero: `base_lane` = table address | lane column, and the address of byte b
-// is base_lane with b in bits 8..15 (one v_perm_b32). `lds0` points at LDS
-// address 0.
-__device__ __forceinline__ u32x4_t nf4_dword_to_bf16_at(const char* lds0, unsigned x,
-                                                        unsigned base_lane, float s) {
-  u32x4_t r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned addr = __builtin_amdgcn_perm(x, base_lane, 0x0C020000u | ((4u + i) << 8));
-    const float2 p = *reinterpret_cast<const float2*>(lds0 + addr);
-    r[i] = bf16x2_bits(p.x * s, p.y * s);
-  }
-  return r;
-}
-
 // ---- exact three-part NF4 codebook (decode kernels) ----
 //
 // Every fp32 codebook value v splits exactly into three bf16 values,
@@ -324,7 +308,9 @@ constexpr int kOOB = (int)0x80000000;  // buffer offset past every resource: loa
 
 // Buffer resources: raw loads through them are bounds-checked by the
 // hardware, so a masked lane gets zeros without a branch (and the compiler
-// keeps exact vmcnt counts for the prefetched loads).
+// keeps exact vmcnt counts for the prefetched loads). The check covers the
+// lane's offset plus the scalar one: the tile kernels' loads rely on it for
+// rows past a tile and behind an expert, their stores for rows past a tile.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int64_t bytes) {
   const int n = bytes < 0x7FFFFFFF ? (int)bytes : 0x7FFFFFFF;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, 0x00020000);

@@ -3654,11 +3654,16 @@ int launch_dgrad(const DgradArgs& p, int block_m, hipStream_t stream,
       const int64_t per_x = tiles_per_xcd(tiles, cus);
       if (per_x * 8 > 0x7FFFFFFF) return -1;
       // Two kernels with the same bits. A 512-column tile of k_tile_dgrad
-      // takes 1.3 (32 rows) to 1.8 (160 rows) times a 256-column tile of
-      // k_dgrad_tall, so it is taken
-      // where it needs at most 5/9 of the rounds of tiles over the CUs
-      // (128 experts, N = 2048, K = 768: 1 against 2 rounds, 75 against 89 us
-      // at 128 rows); with fewer tiles than that, CUs would stand idle.
+      // takes 1.1-1.2 (32 rows) to 1.35-1.55 times (96 and 160 rows) a
+      // 256-column tile of k_dgrad_tall, so rounds of tiles over the CUs
+      // decide; below a round of either, 256 columns keep more CUs at work.
+      // Wide against tall, 32 / 96 / 160 rows (MI355X; NF4 at K = 320, 768,
+      // 1024, 2048, MXFP4 at 2880): 1 against 1 round 1.09-1.20 / 1.25-1.51 /
+      // 1.22-1.53 of the time, 1 against 2 0.60-0.68 / 0.77-0.86 /
+      // 0.80-0.88, 2 against 2 1.16 / 1.44 / 1.43, 2 against 3 0.76-0.83 /
+      // 0.92-1.06 / 0.98-1.11, 3 against 5 0.70-0.73 / 0.89-0.92 / 0.93, 2
+      // against 4 and more at that ratio 0.62-0.65 / 0.75-0.83 / 0.78-0.86.
+      // The line stands on the side where every height gains.
       const int64_t rounds = (tiles + cus - 1) / cus, wide_rounds = (wide + cus - 1) / cus;
       if (block_m <= kDgradWideRows && 9 * wide_rounds <= 5 * rounds) {
         f.t_row0 = p.t_row0;

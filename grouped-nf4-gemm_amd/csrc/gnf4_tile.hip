@@ -23,9 +23,11 @@
 // wave per SIMD issues one instruction in four clocks and waits out every LDS
 // round trip: 3100 clocks per step at 256 rows and 2500 at 32, where the MFMAs
 // need 2048 and 256; this form takes 2330 and 1270 (MXFP4 2310 and 780).
-// What bounds it: at 256 rows the power limit (the clock falls to 1.5 GHz with
-// the matrix cores 88 % busy within the steps), below 100 rows the LDS lookups
-// and the VALU that follow each other in the step.
+// What bounds it: at 256 rows the power limit (283 k clocks per CU in 184 us,
+// 1.5 GHz, where 32 rows run at 2.0; the matrix cores are busy 70 % of all
+// clocks, 88 % within the steps), below 100 rows the LDS lookups and the VALU
+// that follow each other in the step. NF4 takes all 256 registers and spills
+// 24 of them (52 bytes of scratch a lane), none within a tile's step loop.
 // Measured (MI355X, 128 experts, N = 1536, K = 2048, NF4; 32 / 64 / 128 / 256
 // rows per group): 75 / 90 / 118 / 187 us; the four-wave kernel before it 111
 // / 122 / 143 / 215 us. N = 2048, K = 768, 256 rows: 104-107 against 126 us.
@@ -138,8 +140,9 @@ struct WeightLoads {
         u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_of(b, b_bytes), b_voff, g * 32, 0));
   }
   // Scales of steps 4T .. 4T + 3 of F >= 4: a window that ends inside the
-  // row (a resource checks the lane's offset only, not the scalar one added
-  // to it). MXFP4: rows past N read the last row's.
+  // row (the resource spans all of the tile's rows, so it does not keep a
+  // window from running into the next one). MXFP4: rows past N read the last
+  // row's.
   __device__ __forceinline__ ScaleVec<FMT> window(const char* s, int s_bytes, int s_rows,
                                                   int s0) const {
     if constexpr (FMT == kNF4) {

@@ -918,8 +918,8 @@ def _dgrad_block_m(max_rows: int, N: int, K: int) -> int:
 IDS_ARG_MAX = 384
 
 # Tile tables of at most this many m-tiles travel in the kernel arguments of
-# the 256-row kernels (gnf4_hip_grouped_fwd_tiles / _dgrad_tiles): no upload,
-# so no copy is enqueued ahead of the launch (in a captured graph: no copy
+# the persistent tile kernels (gnf4_hip_grouped_fwd_tiles / _dgrad_tiles): no
+# upload, so no copy is enqueued ahead of the launch (in a captured graph: no copy
 # node and no dependency gap before the kernel).
 ARG_TILES_MAX = 256
 
@@ -1014,9 +1014,9 @@ def gemm_4bit_grouped(
 
     Path: groups of at most 16 rows (always when ``max(sizes) == 1``) take the
     decode kernel, which streams each active expert's weights once; larger
-    groups take the tiled MFMA kernel with ``block_m`` (default
-    ``_prefill_block_m(max(sizes))``). An explicit ``block_m`` forces the tiled
-    kernel for groups above one row.
+    groups take the tiled MFMA kernel with tiles of ``block_m`` rows (default:
+    ``_fwd_block_m``; the height changes no bits). An explicit ``block_m``
+    forces the tiled kernel for groups above one row.
 
     The reference's tuning knobs are accepted and validated so call sites keep
     working: ``decode_config`` (BLOCK_N, num_warps), ``split_k`` (>= 1),

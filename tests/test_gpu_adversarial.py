@@ -8,9 +8,9 @@ asks that the codebook x absmax multiply neither flush nor overflow
 differently from the dequant path.
 
 Row counts pick the kernel: 1 row per group runs the fp32 FMA decode path,
-5 and 12 rows the split-codebook MFMA decode (one and two row sets), 40 rows
-the 128-row tiles, 300 rows the 256-row tiles; dgrad runs its 256-row tiles
-and, with K = 96, its 128-row fallback.
+5 and 12 rows the split-codebook MFMA decode (one and two row sets), 40
+and 300 rows the tile kernel (tiles of two and of eight 32-row subtiles); dgrad
+runs its 256-row tiles and, with N = 96, its 128-row fallback.
 """
 import pytest
 import torch
@@ -50,7 +50,7 @@ def test_forward_absmax_extremes(kind, rows):
 @pytest.mark.parametrize("K", [128, 96 * 2])
 def test_dgrad_absmax_extremes(kind, K):
     """dgrad: dX = dY . W with the same absmax extremes; K = 128 runs the
-    four-wave transposed-read tiles, K = 192 with N = 96 (not a multiple of
+    tiles with transposed reads, K = 192 with N = 96 (not a multiple of
     64) the fallback tile kernel."""
     from nf4_grouped import dgrad_4bit_grouped, dequant_ref
     N = 64 if K == 128 else 96

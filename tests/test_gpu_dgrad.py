@@ -126,8 +126,7 @@ def test_dgrad_qwen_down_shape_contract():
 
 @pytest.mark.parametrize("fmt", ["nf4", "mxfp4"])
 def test_dgrad_tall_tiles_and_k_tails(fmt):
-    """Groups above 128 rows run 256-row tiles (the four-wave transposed-read
-    kernel); K = 320 leaves one live 64-column block in the second 256-wide
+    """Groups above 128 rows run 256-row tiles (k_dgrad_tall); K = 320 leaves one live 64-column block in the second 256-wide
     k tile."""
     N, K = 192, 320
     W, S = _stack(fmt, 6, N, K, seed=12)
