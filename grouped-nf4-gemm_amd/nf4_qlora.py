@@ -246,9 +246,9 @@ def _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, n_pack
             and 0 < E <= 65535 and 4 <= r <= 64 and r % 4 == 0 and K % 8 == 0 and N % 8 == 0
             and lora_A.is_contiguous() and lora_B.is_contiguous()
             and lora_A.data_ptr() % 16 == 0 and lora_B.data_ptr() % 16 == 0
-            and T > 0 and sum(int(m) for m in sizes) == T and not _transforming()
+            and T > 0 and sum(sizes) == T and not _transforming()
             and (E >= n_packed or not (torch.is_tensor(expert_ids) and expert_ids.is_cuda)
-                 and all(e < E for e, m in zip(_host_ints(expert_ids), sizes) if int(m) > 0)))
+                 and all(e < E for e, m in zip(_host_ints(expert_ids), sizes) if m > 0)))
 
 
 # Rows of a chunk of gnf4_hip_lora_wgrad_split
@@ -260,40 +260,39 @@ class _LoraTables:
     of the caller's is kept: it may write the next layer's routing into the
     same tensor or list before backward."""
 
-    def __init__(self, sizes, expert_ids, dev):
-        self.sizes = [int(v) for v in sizes]
-        m = np.asarray(self.sizes, dtype=np.int32)
-        off = np.zeros((3, len(m) + 1), dtype=np.int32)
+    def __init__(self, sizes, expert_ids, dev, E):
+        self.sizes, self.G = sizes, len(sizes)   # (a list of ints of its own)
+        on_dev = torch.is_tensor(expert_ids) and expert_ids.is_cuda
+        ids = [] if on_dev else [nf4_grouped._np_ids(expert_ids).copy()]
+        m = np.asarray(sizes, dtype=np.int32)
+        most = max(sizes)   # rows of the largest expert (device ids: group)
+        if not on_dev and len(set(ids[0].tolist())) < self.G:
+            most = int(np.bincount(ids[0], m).max())
+        # Whether the adapter gradients take the kernel that splits an
+        # expert's rows over waves: where one wave per expert would run long
+        # (from 384 rows) while other waves idle (fewer than 32 such experts'
+        # worth of rows). Direct and split, MI355X, K = 2048, r = 16, even
+        # groups: 8 experts of 320 / 384 / 512 / 4096 rows 25 / 29 / 38 / 328
+        # and 23 / 23 / 24 / 46 us; 32 experts of 320 / 384 / 1024 31 / 36 / 88
+        # and 31 / 32 / 44 us; 64 experts of 384 / 512 / 1024 39 / 50 / 101 and
+        # 45 / 45 / 75 us, at r = 64 90 / 113 / 211 and 132 / 133 / 275 us.
+        # More device ids than experts: some are repeated, so it splits.
+        self.split = most >= 384 and 32 * most >= sum(sizes) or self.G > E
+        off = np.zeros((3 if self.split else 2, self.G + 1), dtype=np.int32)
         np.cumsum((m + 15) // 16, out=off[0, 1:])
         np.cumsum(m, out=off[1, 1:])
-        np.cumsum((m + _WGRAD_CHUNK - 1) // _WGRAD_CHUNK, out=off[2, 1:])
-        on_dev = torch.is_tensor(expert_ids) and expert_ids.is_cuda
-        ids = [] if on_dev else [nf4_grouped._np_ids(expert_ids)]
+        if self.split:
+            np.cumsum((m + _WGRAD_CHUNK - 1) // _WGRAD_CHUNK, out=off[2, 1:])
+            self.n_chunks = int(off[2, -1])
         views = nf4_grouped.to_device_i32([*off, *ids], dev)
-        self.n, self.G = int(off[0, -1]), len(m)
-        self.n_chunks = int(off[2, -1])
-        self.tile_off, self.row_off, self.chunk_off = views[:3]
+        self.n = int(off[0, -1])
+        self.tile_off, self.row_off = views[:2]
+        self.chunk_off = views[2] if self.split else None
         self.ids = (torch.empty(self.G, dtype=torch.int32, device=dev).copy_(expert_ids)
-                    if on_dev else views[3])
-        self.expert_ids = self.ids if on_dev else ids[0].tolist()   # for the composition
-        # the most rows an expert has (device ids: of one group)
-        self.most = int(m.max() if on_dev else np.bincount(ids[0], m).max())
-
-    def split_rows(self, E) -> bool:
-        """Whether the adapter gradients take the kernel that splits an
-        expert's rows over waves: where one wave per expert would run long
-        (from 384 rows) while other waves idle (fewer than 32 such experts'
-        worth of rows). Direct and split, MI355X, K = 2048, r = 16, even
-        groups: 8 experts of 320 / 384 / 512 / 4096 rows 25 / 29 / 38 / 328
-        and 23 / 23 / 24 / 46 us; 32 experts of 320 / 384 / 1024 31 / 36 / 88
-        and 31 / 32 / 44 us; 64 experts of 384 / 512 / 1024 39 / 50 / 101 and
-        45 / 45 / 75 us, at r = 64 90 / 113 / 211 and 132 / 133 / 275 us. More
-        device ids than experts: some are repeated, so it splits."""
-        return self.most >= 384 and 32 * self.most >= sum(self.sizes) or self.G > E
-
-    def args(self):
-        return (self.tile_off.data_ptr(), self.row_off.data_ptr(), self.ids.data_ptr(), self.G,
-                self.n)
+                    if on_dev else views[-1])
+        self.expert_ids = self.ids if on_dev else ids[0]   # for the composition
+        self.args = (self.tile_off.data_ptr(), self.row_off.data_ptr(), self.ids.data_ptr(),
+                     self.G, self.n)
 
 
 def _rows(t):
@@ -307,41 +306,46 @@ def _rows(t):
     return t
 
 
-def _lora_call(name, dev, *args):
-    with nf4_grouped._device_ctx(dev):
-        rc = getattr(_hiplib.load(), name)(*args, nf4_grouped._stream_ptr(dev))
-    _hiplib.check(rc, "fused_grouped_lora")
+class _Launches:
+    """The LoRA launches of one direction: the library and the current stream
+    of a device, looked up once."""
+
+    def __init__(self, dev):
+        self.lib = _hiplib.load()
+        self.stream = nf4_grouped._stream_ptr(dev)
+
+    def __call__(self, name, *args):
+        _hiplib.check(getattr(self.lib, name)(*args, self.stream), "fused_grouped_lora")
 
 
-def _lora_down(x, w, transposed, tb, scale, r):
+def _lora_down(call, x, w, transposed, tb, scale, r):
     E, C = w.shape[0], x.shape[1]
     y = torch.empty(x.shape[0], r, dtype=torch.float32, device=x.device)
-    _lora_call("gnf4_hip_lora_down", x.device, x.data_ptr(), x.stride(0), w.data_ptr(),
-               transposed, E, C, r, *tb.args(), scale, y.data_ptr())
+    call("gnf4_hip_lora_down", x.data_ptr(), x.stride(0), w.data_ptr(), transposed, E, C, r,
+         *tb.args, scale, y.data_ptr())
     return y
 
 
-def _lora_up(u, w, transposed, C, tb, scale, base=None):
+def _lora_up(call, u, w, transposed, C, tb, scale, base=None):
     T, r = u.shape
     out = torch.empty(T, C, dtype=torch.bfloat16, device=u.device)
-    _lora_call("gnf4_hip_lora_up", u.device, u.data_ptr(), w.data_ptr(), transposed, w.shape[0],
-               C, r, *tb.args(), scale, base.data_ptr() if base is not None else None,
-               base.stride(0) if base is not None else 0, out.data_ptr(), out.stride(0))
+    call("gnf4_hip_lora_up", u.data_ptr(), w.data_ptr(), transposed, w.shape[0], C, r, *tb.args,
+         scale, base.data_ptr() if base is not None else None,
+         base.stride(0) if base is not None else 0, out.data_ptr(), out.stride(0))
     return out
 
 
-def _lora_wgrad(p, q, like, transposed, tb, scale):
+def _lora_wgrad(call, p, q, like, transposed, tb, scale):
     dw = torch.empty_like(like)
     E, C, r = like.shape[0], p.shape[1], q.shape[1]
-    if tb.split_rows(E):
+    if tb.split:
         part = torch.empty(tb.n_chunks, C * r, dtype=torch.float32, device=p.device)
-        _lora_call("gnf4_hip_lora_wgrad_split", p.device, p.data_ptr(), p.stride(0), q.data_ptr(),
-                   transposed, E, C, r, tb.chunk_off.data_ptr(), tb.row_off.data_ptr(),
-                   tb.ids.data_ptr(), tb.G, tb.n_chunks, scale, part.data_ptr(), dw.data_ptr())
+        call("gnf4_hip_lora_wgrad_split", p.data_ptr(), p.stride(0), q.data_ptr(), transposed, E,
+             C, r, tb.chunk_off.data_ptr(), tb.row_off.data_ptr(), tb.ids.data_ptr(), tb.G,
+             tb.n_chunks, scale, part.data_ptr(), dw.data_ptr())
         return dw
-    _lora_call("gnf4_hip_lora_wgrad", p.device, p.data_ptr(), p.stride(0), q.data_ptr(),
-               transposed, E, C, r, tb.ids.data_ptr(), tb.row_off.data_ptr(), tb.G, scale,
-               dw.data_ptr())
+    call("gnf4_hip_lora_wgrad", p.data_ptr(), p.stride(0), q.data_ptr(), transposed, E, C, r,
+         tb.ids.data_ptr(), tb.row_off.data_ptr(), tb.G, scale, dw.data_ptr())
     return dw
 
 
@@ -366,9 +370,11 @@ class _LoraAdd(torch.autograd.Function):
         if recording:
             a_cat, lora_A, lora_B = a_cat.clone(), lora_A.clone(), lora_B.clone()
         a = _rows(a_cat.detach())
-        tb = _LoraTables(sizes, expert_ids, a.device)
-        u = _lora_down(a, lora_A, 0, tb, 1.0, lora_A.shape[1])
-        out = _lora_up(u, lora_B, 0, lora_B.shape[1], tb, float(scaling), _rows(base))
+        tb = _LoraTables(sizes, expert_ids, a.device, lora_A.shape[0])
+        with nf4_grouped._device_ctx(a.device):
+            call = _Launches(a.device)
+            u = _lora_down(call, a, lora_A, 0, tb, 1.0, lora_A.shape[1])
+            out = _lora_up(call, u, lora_B, 0, lora_B.shape[1], tb, float(scaling), _rows(base))
         if not recording:
             return out
         ctx.set_materialize_grads(False)
@@ -395,11 +401,17 @@ class _LoraAdd(torch.autograd.Function):
             grads = [next(got) if n else None for n in need[1:4]]
         else:
             s = float(scaling)
-            gv = _rows(g)
-            gu = _lora_down(gv, B, 1, tb, s, A.shape[1]) if need[1] or need[2] else None
-            ga = _lora_up(gu, A, 1, a_cat.shape[1], tb, 1.0) if need[1] else None
-            gA = _lora_wgrad(_rows(a_cat), gu, A, 1, tb, 1.0) if need[2] else None
-            gB = _lora_wgrad(gv, u, B, 0, tb, s) if need[3] else None
+            ga = gA = gB = gu = None
+            with nf4_grouped._device_ctx(g.device):
+                call, gv = _Launches(g.device), _rows(g)
+                if need[1] or need[2]:
+                    gu = _lora_down(call, gv, B, 1, tb, s, A.shape[1])
+                if need[1]:
+                    ga = _lora_up(call, gu, A, 1, a_cat.shape[1], tb, 1.0)
+                if need[2]:
+                    gA = _lora_wgrad(call, _rows(a_cat), gu, A, 1, tb, 1.0)
+                if need[3]:
+                    gB = _lora_wgrad(call, gv, u, B, 0, tb, s)
             grads = [ga, gA, gB]
         grads = [x if y is None else y if x is None else x + y for x, y in zip(grads, g_copies)]
         return (g, *grads, None, None, None, None)
@@ -414,8 +426,9 @@ def fused_grouped_lora(a_cat, packed, absmax, sizes, expert_ids, lora_A=None, lo
                                   weights_fn=weights_fn, dgrad_kernel=dgrad_kernel)
     if lora_A is None or lora_B is None:
         return out
-    if _kernels_take(out, a_cat, lora_A, lora_B, sizes, scaling, expert_ids, packed.shape[0]):
-        out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, sizes, expert_ids, scaling,
+    rows = [int(m) for m in sizes]
+    if _kernels_take(out, a_cat, lora_A, lora_B, rows, scaling, expert_ids, packed.shape[0]):
+        out = _LoraAdd.apply(out, a_cat, lora_A, lora_B, rows, expert_ids, scaling,
                              torch.is_grad_enabled())
         return out[0] if isinstance(out, tuple) else out
     delta = lora_delta_grouped(a_cat, lora_A, lora_B, sizes, expert_ids, scaling)

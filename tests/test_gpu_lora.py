@@ -281,8 +281,9 @@ def test_adapter_gradients_of_long_groups(sizes, ids, E, K, N, r, split, dev_ids
     if dev_ids and max(sizes) < 384:
         split = len(ids) > E
     names = []
-    orig = nf4_qlora._lora_call
-    monkeypatch.setattr(nf4_qlora, "_lora_call", lambda n, *a: names.append(n) or orig(n, *a))
+    orig = nf4_qlora._Launches.__call__
+    monkeypatch.setattr(nf4_qlora._Launches, "__call__",
+                        lambda self, n, *a: names.append(n) or orig(self, n, *a))
     _out, _gx, gA, gB = _run(True, W, S, x, A, B, go, sizes, arg, monkeypatch)
     assert names.count("gnf4_hip_lora_wgrad_split") == (2 if split else 0)
     assert names.count("gnf4_hip_lora_wgrad") == (0 if split else 2)
