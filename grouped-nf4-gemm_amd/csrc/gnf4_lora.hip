@@ -15,11 +15,12 @@
 // each lane's global accesses are 16 contiguous bytes.
 //
 // Measured (MI355X, 8192 rows, 128 experts, K = 2048, N = 1536, r = 16): u
-// and gu 23 and 18 us (34 and 25 MB of rows: 1.5 TB/s, from the latency of few
+// and gu 23 and 18 us (34 and 25 MB of rows: 1.4 TB/s, from the latency of few
 // loads per wave), out and gx 24 us each (50 and 34 MB, 2.1 and 1.4 TB/s), gA
-// and gB 18 and 13 us. With gathers, padding to the widest group, batched fp32
-// products and index scatters the same parts took about 900 us; the whole
-// training pass through the projection went from 1156 to 468 us.
+// and gB 17 and 14 us (2.0 and 1.8 TB/s). With gathers, padding to the widest
+// group, batched fp32 products and index scatters the same parts took about
+// 900 us; the whole training pass through the projection went from 1151 to
+// 524 us (358 us of kernels, 26 of them the copies its backward reads).
 
 #include "gnf4_device.h"
 

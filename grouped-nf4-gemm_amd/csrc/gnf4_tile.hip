@@ -22,7 +22,8 @@
 // Why eight waves of 32 rows and not four of 64 (half the operand reads): one
 // wave per SIMD issues one instruction in four clocks and waits out every LDS
 // round trip: 3100 clocks per step at 256 rows and 2500 at 32, where the MFMAs
-// need 2048 and 256; this form takes 2330 and 1270 (MXFP4 2310 and 780).
+// need 2048 and 256; this form takes 2330 and 1270 (MXFP4 2310 and 780; clock
+// stamps in a measuring build).
 // What bounds it: at 256 rows the power limit (283 k clocks per CU in 184 us,
 // 1.5 GHz, where 32 rows run at 2.0; the matrix cores are busy 70 % of all
 // clocks, 88 % within the steps), below 100 rows the LDS lookups and the VALU
