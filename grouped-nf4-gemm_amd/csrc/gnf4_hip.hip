@@ -460,7 +460,9 @@ __device__ __forceinline__ void decode_unit(const FwdArgs& p, const int g, const
               c[s][j & 1] = mfma(a[s][j], lo, c[s][j & 1]);
             }
           }
-          const float am = __uint_as_float(sb[i][t]);
+          // (past the end of K the run's absmax load holds the next row's or
+          // padding: zeros times those need not be zero)
+          const float am = kval ? __uint_as_float(sb[i][t]) : 0.0f;
 #pragma unroll
           for (int s = 0; s < kSets; ++s)
 #pragma unroll
@@ -1592,7 +1594,9 @@ __global__ void __launch_bounds__(1024, 1)
         for (int t = 0; t < kT; ++t) {
           const int idx = 2 * i + (q >> 1);
           const u32x4_t v = sq[slot][t];
-          const float am = __uint_as_float(idx == 0 ? v[0] : idx == 1 ? v[1] : idx == 2 ? v[2] : v[3]);
+          const unsigned sbits = idx == 0 ? v[0] : idx == 1 ? v[1] : idx == 2 ? v[2] : v[3];
+          // past the end of K: not this row's absmax
+          const float am = kseg < (unsigned)K32 ? __uint_as_float(sbits) : 0.0f;
           f32x4_t c[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {

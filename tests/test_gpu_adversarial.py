@@ -15,7 +15,7 @@ runs its 256-row tiles and, with N = 96, its 128-row fallback.
 import pytest
 import torch
 
-from _fixtures import dequant, fp64_ref, rel_err
+from _fixtures import dequant, fp64_ref, rand_acts, rand_nf4_stack, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +84,42 @@ def test_single_block_outlier(rows):
     ref = a.double() @ dequant("nf4", B[0], A[0]).double().t()
     err = (out.double() - ref).abs().max() / ref.abs().max().clamp_min(1e-4)
     assert err < 1e-2
+
+
+@pytest.mark.parametrize("K", [64, 192, 320, 1088, 1152, 1984, 2880])
+@pytest.mark.parametrize("sizes", [[1, 1, 1], [2, 1, 2], [4, 3, 1], [8, 5, 2], [12, 1, 9],
+                                   [40, 3, 20], [8] * 64])
+def test_scales_behind_a_row_do_not_reach_it(K, sizes):
+    """The kernels load absmax values in pairs of 128-element chunks: past the
+    end of a row they hold the next row's, or what pads it. Infinities in
+    every second row's scales, and NaN as padding, leave the other rows' bits
+    alone, in every launch class (K a multiple of 128 or not)."""
+    from nf4_grouped import gemm_4bit_grouped
+    N, E = 1536 if len(sizes) > 3 else 72, 3
+    B, S = rand_nf4_stack(E, N, K, seed=9)
+    ids = [i % E for i in range(len(sizes))]
+    a = rand_acts(sum(sizes), K, seed=10)
+    want = gemm_4bit_grouped(a, B, S, sizes, ids)
+    wild = S.clone()
+    wild[:, 1::2] = float("inf")
+    assert torch.equal(gemm_4bit_grouped(a, B, wild, sizes, ids)[:, ::2], want[:, ::2])
+    buf = torch.full((E, N, S.shape[2] + 3), float("nan"), device="cuda")
+    buf[..., :S.shape[2]] = S
+    assert torch.equal(gemm_4bit_grouped(a, B, buf[..., :S.shape[2]], sizes, ids), want)
+
+
+@pytest.mark.parametrize("H,K", [(64, 192), (320, 1088), (192, 2880)])
+def test_scales_behind_a_row_do_not_reach_it_in_the_fused_ffn(H, K):
+    from nf4_ffn import gemm_nf4_ffn_grouped
+    gu, dn = rand_nf4_stack(3, 2 * H, K, seed=11), rand_nf4_stack(3, K, H, seed=12)
+
+    def padded(S):
+        buf = torch.full((*S.shape[:2], S.shape[2] + 3), float("nan"), device="cuda")
+        buf[..., :S.shape[2]] = S
+        return buf[..., :S.shape[2]]
+
+    for sizes in ([1, 1], [3, 2], [8, 1], [12, 9]):
+        a = rand_acts(sum(sizes), K, seed=13)
+        want = gemm_nf4_ffn_grouped(a, *gu, *dn, sizes, [2, 0])
+        got = gemm_nf4_ffn_grouped(a, gu[0], padded(gu[1]), dn[0], padded(dn[1]), sizes, [2, 0])
+        assert torch.equal(got, want)
